@@ -88,9 +88,11 @@ int mt_paged_decode_batch_noalloc(void* out, const void* q, const void* k, const
 
 /* Number of launches since the library was loaded in which
  * mt_paged_attention / mt_paged_prefill split one long prompt's keys over
- * workgroups (query tiles x heads <= compute units, >= 6 key blocks in the
- * last tile). A diagnostic, e.g. for tests that must exercise that path.
- * No reference counterpart. */
+ * wave groups or workgroups because the prompt alone leaves compute units idle
+ * (64-query tiles x heads <= compute units, >= 6 key blocks of 64 in the last
+ * tile), and of mt_paged_prefill_ragged launches whose longest tile spans at
+ * least 6 key blocks and more than its share of the launch. A diagnostic, e.g.
+ * for tests that must exercise that path. No reference counterpart. */
 int mt_paged_prefill_key_splits(long long* launches);
 
 /* Bytes of workspace mt_paged_decode_split needs (0 when no row can be split).
@@ -154,8 +156,9 @@ int mt_paged_decode_split(void* out, const void* q, const void* k, const void* v
  * q, k and v are [b, n, qkv_stride] with head j at columns [j*d, (j+1)*d)
  * (qkv_stride = 3*h*d when they are column blocks of one fused projection;
  * 0 = h*d) and out is [b, n, out_stride] with heads merged the same way
- * (0 = h*d). The matrix-core kernel serves fp16/bf16 with d 64 or 128 and
- * n >= 16. No reference counterpart as one entry (reference
+ * (0 = h*d). The matrix-core kernel serves n >= 2 with rows of whole 16-byte
+ * chunks (d a multiple of 8 in fp16/bf16, of 4 in fp32) at 16-byte aligned
+ * addresses. No reference counterpart as one entry (reference
  * paged_kv_cache.py:205-221 calls mt_paged_append and mt_paged_attention on
  * head-split copies). */
 int mt_paged_prefill(void* out, const void* q, const void* k, const void* v, const uint64_t* slabs,
@@ -169,8 +172,8 @@ int mt_paged_prefill(void* out, const void* q, const void* k, const void* v, con
  * offset offsets[r] and its own block-table row tables[r] (a device pointer
  * to `columns` entries); tables, tokens and offsets are host arrays. Each
  * prompt's K/V are appended and its causal attention computed as
- * mt_paged_prefill would; with fp16/bf16, d 64/128 and 16-byte rows, up to 16
- * prompts (256 query tiles) share one append and one matrix-core launch.
+ * mt_paged_prefill would; with rows of whole 16-byte chunks up to 16 prompts
+ * (256 tiles of 64 queries) share one append and one matrix-core launch.
  * No reference counterpart (the reference prefills one request per call). */
 int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void* v,
                             const uint64_t* slabs, const int* const* tables, const int* tokens,

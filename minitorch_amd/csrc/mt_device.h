@@ -34,9 +34,7 @@ __device__ __forceinline__ uint16_t f32_to_f16(float x) {
   return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x));
 }
 __device__ __forceinline__ uint16_t f32_to_bf16(float x) {
-  uint32_t u = __float_as_uint(x);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-  return static_cast<uint16_t>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(x));  // one v_cvt_pk_bf16_f32
 }
 
 template <int DT> __device__ __forceinline__ float to_f32(typename Elem<DT>::T x) {
@@ -80,6 +78,18 @@ template <int DT> __device__ __forceinline__ u32x4 pack16(const float* v) {
     r.x = w[0]; r.y = w[1]; r.z = w[2]; r.w = w[3];
   }
   return r;
+}
+
+// Stores four consecutive values (16-byte aligned in fp32, 8-byte in
+// fp16/bf16).
+template <int DT>
+__device__ __forceinline__ void store4(typename Elem<DT>::T* p, float a, float b, float c, float d) {
+  if constexpr (DT == kF32)
+    *reinterpret_cast<float4*>(p) = float4{a, b, c, d};
+  else
+    *reinterpret_cast<uint2*>(p) =
+        uint2{static_cast<uint32_t>(from_f32<DT>(a)) | (static_cast<uint32_t>(from_f32<DT>(b)) << 16),
+              static_cast<uint32_t>(from_f32<DT>(c)) | (static_cast<uint32_t>(from_f32<DT>(d)) << 16)};
 }
 
 template <int DT> constexpr int per16() { return 16 / elem_bytes<DT>(); }

@@ -32,9 +32,9 @@
 //     separate launch.)
 //
 // Causal attention of several queries per request (a prefill) runs on the
-// matrix cores for fp16/bf16 (prefill_kernel: 64-query tiles, S^T = K Q^T and
-// O^T += V^T P^T with v_mfma_f32_16x16x32); fp32 and the shapes it does not
-// take use the per-query query_kernel.
+// matrix cores for every type and head dims of whole 16-byte chunks
+// (causal_kernel: 32 queries a wave, S^T = K Q^T and O^T += V^T P^T); a single
+// query and the shapes it does not take use the per-query query_kernel.
 #include "mt_device.h"
 #include "../../include/mt_paged.h"
 #include <algorithm>
@@ -49,6 +49,7 @@
 #endif
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 using namespace mt;
@@ -1257,102 +1258,137 @@ struct AppendArgs {
 
 
 // ---------------------------------------------------------------------------
-// Causal paged prefill attention on the matrix cores (fp16/bf16, head_dim 64
-// or 128), same semantics as query_kernel: query qi attends keys
-// kj < nk with kj <= offset + qi, and a query whose keys touch a missing page
-// reads NaN. One workgroup of 4 waves per (request, head, 64-query tile),
-// each wave owning 16 queries; keys stream in blocks of 64 staged in LDS from
-// the pages (K row-major, V transposed). Per block a wave computes
-// S^T = K Q^T with v_mfma_f32_16x16x32 (keys x queries, so each lane holds 16
-// scores of one query), updates that query's online softmax in registers and
-// accumulates O^T += V^T P^T, feeding the scores' own register layout as the
-// B operand (the MFMA sums over its k index in any order, so A's key order is
-// chosen to match). The MFMA takes P in the input type, so P is split into a
-// high and a low part of that type (two MFMAs): the weights keep about 16
-// (bf16) or 22 (fp16) significant bits instead of 8 or 11, which holds the
-// output to the fp32 path's accuracy when |V| is large.
-constexpr int kPfQueries = 64;     // queries per workgroup
-constexpr int kPfKeys = 64;        // keys per staged block
+// Causal paged attention of several queries per request on the matrix cores,
+// same semantics as query_kernel: query qi attends keys kj < nk with
+// kj <= offset + qi, and a query whose keys touch a missing page reads NaN.
+//
+// A workgroup owns a tile of 32 QT queries of one (request, head). It has
+// QT x KG waves: wave (qt, kg) holds 32 of the tile's queries and takes every
+// KG-th block of KB keys; the KG groups' softmax states meet in LDS at the
+// end. A staged round is KG blocks, copied from the pages (or from the
+// prompt's own K/V rows) to LDS by all waves while the round before it is
+// computed.
+//
+// Per block a wave computes S^T = K Q^T with 32x32 MFMAs (keys x queries, so
+// two lanes share a query and each holds half of the block's scores of it),
+// updates that query's online softmax in registers and accumulates
+// O^T += V^T P^T, feeding the scores' own register layout as the B operand
+// (the MFMA sums over its k index in any order, so A's key order is chosen to
+// match). K and V both lie row-major in LDS; for 16-bit types V's operand is
+// read transposed by ds_read_b64_tr_b16, for fp32 a lane reads single
+// elements. Rows are swizzled in 16-byte chunks so that these reads are free
+// of bank conflicts. Rounds go from memory to LDS without passing through
+// registers, so that a wave's registers hold its queries, scores and output:
+// two to four waves per SIMD, which is what the kernel lives on. Its bound is
+// the issue of a block's ~170 VALU instructions (exponentials, the split of
+// P) between 12 MFMAs; rounds deeper in flight, and all loads through
+// registers, measured the same or slower. Against the 16-query waves with V
+// transposed by 2-byte LDS stores that it replaces (us per call, bf16): 2048
+// tokens at offset 2048 x 16 heads 60 against 134 (430 against 192 TFLOP/s),
+// 1000 tokens x 16 heads 15.2 against 22.7, 16 prompts of 32-512 tokens x 12
+// heads fp16 19.8 against 26.3; fp32, which query_kernel read K/V for once per
+// query: 4 x 333 tokens x 12 heads 20 against 106.
+//
+// For fp16/bf16 the MFMA takes P in the input type, so P is split into a high
+// and a low part of that type (two MFMAs): the weights keep about 16 (bf16)
+// or 22 (fp16) significant bits instead of 8 or 11, which holds the output to
+// the fp32 path's accuracy when |V| is large. fp32 runs on the fp32 MFMA
+// (v_mfma_f32_32x32x2_f32), nothing is rounded below fp32.
+//
+// The running reference of the exponentials moves only when a score exceeds
+// it by kRescale (base 2), so most blocks skip the rescaling of O: weights
+// are then at most 2^kRescale, which neither fp32 nor the hi/lo split minds.
 constexpr int kPfWindowPages = 512;  // page bases resolved into LDS at a time
-#ifndef MT_PREFILL_MIN_QUERIES
-#define MT_PREFILL_MIN_QUERIES 16
-#endif
-constexpr int kPfMinQueries = MT_PREFILL_MIN_QUERIES;  // fewer queries use query_kernel
+constexpr int kPfBlock = 64;         // keys per unit of a split over workgroups
+constexpr float kRescale = 6.f;
+constexpr int kPfMinQueries = 2;     // fewer queries use query_kernel
 
-// x of lane l ^ 16 and of lane l ^ 32, combined with x by the caller: the
-// permlane swaps exchange rows of 16 (32) lanes between two registers, so
-// after swapping two copies of x, lane l holds x[l] in one and x[l ^ 16]
-// (x[l ^ 32]) in the other.
-__device__ __forceinline__ float lane_swap16(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  const float a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-  return (threadIdx.x & 16) ? a : b;
-}
-__device__ __forceinline__ float lane_swap32(float x) {
+// x of lanes l and l ^ 32 (in either order): the permlane swap of two copies
+// of x leaves x[l % 32] in one and x[l % 32 + 32] in the other.
+__device__ __forceinline__ float max_halves(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  const float a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-  return (threadIdx.x & 32) ? a : b;
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float add_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Two probabilities rounded to the input type, packed as the MFMA operand;
-// r0/r1 receive the rounded values as floats (for the low part of the split).
-// fp16 rounds toward zero (one packed conversion; the low part carries the
-// remainder), bf16 to nearest even.
+// Two probabilities as the high and low packed MFMA operands: hi = p rounded
+// to the input type (fp16 toward zero, one packed conversion; bf16 to nearest
+// even), lo = the remainder, rounded the same way.
 template <int DT>
-struct PackP;
+struct SplitP;
 template <>
-struct PackP<kF16> {
-  static __device__ __forceinline__ uint32_t pack(float p0, float p1, float& r0, float& r1) {
+struct SplitP<kF16> {
+  static __device__ __forceinline__ void split(float p0, float p1, uint32_t& hi, uint32_t& lo) {
     const auto h = __builtin_amdgcn_cvt_pkrtz(p0, p1);
-    r0 = float(h[0]);
-    r1 = float(h[1]);
-    return __builtin_bit_cast(uint32_t, h);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p0 - float(h[0]), p1 - float(h[1])));
   }
 };
 template <>
-struct PackP<kBF16> {
+struct SplitP<kBF16> {
   typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-  static __device__ __forceinline__ uint32_t pack(float p0, float p1, float& r0, float& r1) {
+  static __device__ __forceinline__ void split(float p0, float p1, uint32_t& hi, uint32_t& lo) {
     const bf2 h = {static_cast<__bf16>(p0), static_cast<__bf16>(p1)};
-    const uint32_t u = __builtin_bit_cast(uint32_t, h);
-    r0 = __uint_as_float(u << 16);
-    r1 = __uint_as_float(u & 0xffff0000u);
-    return u;
+    hi = __builtin_bit_cast(uint32_t, h);
+    asm("" : "+v"(hi));  // keeps the halves' unpacking from becoming two more conversions
+    const float r0 = p0 - __uint_as_float(hi << 16), r1 = p1 - __uint_as_float(hi & 0xffff0000u);
+    const bf2 r = {static_cast<__bf16>(r0), static_cast<__bf16>(r1)};
+    lo = __builtin_bit_cast(uint32_t, r);
   }
 };
 
-// What one prefill workgroup works on: query tile `tile` of `head` of a
-// request whose queries start at element q0 of q (o0 of out), nq queries at
-// key offset `offset` over the pages of table_row.
+// What one workgroup works on: query tile `tile` of `head` of a request whose
+// queries start at element q0 of q (o0 of out), nq queries at key offset
+// `offset` over the pages of table_row.
 struct PfItem {
   int tile, head, nq, offset;
   int64_t q0, o0;
   const int* table_row;
-  int kb0, kb1;  // key blocks [kb0, kb1) of the tile's keys that this item attends
+  int kb0, kb1;  // kPfBlock-key blocks [kb0, kb1) of the tile's keys that this item attends
   int slot;      // partials slot of a split tile, -1: the item writes the output rows
 };
 
 constexpr int kAllKeyBlocks = 1 << 24;
 
+// Blocks of kPfBlock keys that query tile `tile` (tq queries a tile) attends.
+__host__ __device__ __forceinline__ int key_blocks(int tile, int tq, int nq, int offset) {
+  const int64_t end = int64_t(tile + 1) * tq < nq ? int64_t(tile + 1) * tq : nq;
+  return int((offset + end + kPfBlock - 1) / kPfBlock);
+}
+
 // The uniform batch of QueryArgs (b requests of nq queries at one offset):
-// items ordered by tile, last (longest) tiles first.
+// items ordered by tile, last (longest) tiles first. With `share` > 0 each
+// tile's keys are cut into pieces of at most `share` blocks, at most `pieces`
+// per tile (a tile with one piece writes its output rows).
 struct UniformItems {
+  int tiles, pieces, share;
   __device__ __forceinline__ int64_t count(const QueryArgs& a) const { return a.items; }
-  __device__ __forceinline__ PfItem get(int64_t item, const QueryArgs& a) const {
-    const int tiles = (a.nq + kPfQueries - 1) / kPfQueries;
-    const int64_t bh_count = a.items / tiles;
-    PfItem it;
-    it.tile = tiles - 1 - int(item / bh_count);
-    const int64_t bh = item - int64_t(tiles - 1 - it.tile) * bh_count;
-    const int b = int(bh / a.g.heads);
-    it.head = int(bh - int64_t(b) * a.g.heads);
+  __device__ __forceinline__ bool get(int64_t item, const QueryArgs& a, int tq, PfItem& it) const {
+    const unsigned bh_count = unsigned(a.batch) * unsigned(a.g.heads);
+    const unsigned tp = unsigned(item) / bh_count;  // (tile, piece), from the last tile down
+    const unsigned bh = unsigned(item) - tp * bh_count;
+    const unsigned t = tp / unsigned(pieces);
+    const int piece = int(tp - t * unsigned(pieces));
+    const int b = int(bh / unsigned(a.g.heads));
+    it.tile = tiles - 1 - int(t);
+    it.head = int(bh) - b * a.g.heads;
     it.nq = a.nq;
     it.offset = a.offset;
     it.q0 = b * a.q_b + it.head * a.q_h;
     it.o0 = b * a.o_b + it.head * a.o_h;
     it.table_row = a.table + int64_t(b) * a.g.columns;
     it.kb0 = 0; it.kb1 = kAllKeyBlocks; it.slot = -1;
-    return it;
+    if (pieces > 1) {
+      const int nb = key_blocks(it.tile, tq, it.nq, it.offset);
+      it.kb0 = piece * share;
+      it.kb1 = it.kb0 + share < nb ? it.kb0 + share : nb;
+      if (nb > share) it.slot = (b * tiles + it.tile) * pieces + piece;
+      return it.kb0 < nb;
+    }
+    return true;
   }
 };
 
@@ -1360,12 +1396,6 @@ struct UniformItems {
 // rows [first_row[r], first_row[r] + n[r]) of q/k/v/out, with its own table
 // row and key offset), passed by value: every (prompt, tile) pair in the
 // order of pair_prompt / pair_tile (heaviest first), times the heads.
-#ifndef MT_RAGGED_SHARE
-#define MT_RAGGED_SHARE 2  // workgroups per compute unit that a ragged launch's key blocks are shared over
-#endif
-#ifndef MT_RAGGED_KEY_SPLIT
-#define MT_RAGGED_KEY_SPLIT 1
-#endif
 constexpr int kRaggedPrompts = 16;
 constexpr int kRaggedTiles = 256;
 struct RaggedItems {
@@ -1379,12 +1409,11 @@ struct RaggedItems {
   unsigned short pair_kb0[kRaggedTiles], pair_kb1[kRaggedTiles];
   short pair_slot[kRaggedTiles];
   __device__ __forceinline__ int64_t count(const QueryArgs& a) const { return int64_t(pairs) * a.g.heads; }
-  __device__ __forceinline__ PfItem get(int64_t item, const QueryArgs& a) const {
-    const int p = int(item / a.g.heads);
+  __device__ __forceinline__ bool get(int64_t item, const QueryArgs& a, int, PfItem& it) const {
+    const int p = int(unsigned(item) / unsigned(a.g.heads));
     const int r = pair_prompt[p];
-    PfItem it;
     it.tile = pair_tile[p];
-    it.head = int(item - int64_t(p) * a.g.heads);
+    it.head = int(item) - p * a.g.heads;
     it.nq = n[r];
     it.offset = offset[r];
     it.q0 = int64_t(first_row[r]) * a.q_r + it.head * a.q_h;
@@ -1393,305 +1422,497 @@ struct RaggedItems {
     it.slot = pair_slot[p];
     it.kb0 = it.slot >= 0 ? pair_kb0[p] : 0;
     it.kb1 = it.slot >= 0 ? pair_kb1[p] : kAllKeyBlocks;
-    return it;
+    return true;
   }
 };
 
-// One request (QueryArgs with batch 1) whose long query tiles have their
-// keys split over several workgroups: (tile, key blocks [kb0, kb1), slot)
-// per pair, heaviest first, times the heads. A tile with one split writes its
-// output; the splits of the others write partials for prefill_merge_kernel.
-constexpr int kSplitPairs = 256;
-struct SplitItems {
-  int pairs;
-  unsigned short tile[kSplitPairs], kb0[kSplitPairs], kb1[kSplitPairs];
-  short slot[kSplitPairs];
-  __device__ __forceinline__ int64_t count(const QueryArgs& a) const { return int64_t(pairs) * a.g.heads; }
-  __device__ __forceinline__ PfItem get(int64_t item, const QueryArgs& a) const {
-    const int p = int(item / a.g.heads);
-    PfItem it;
-    it.tile = tile[p];
-    it.head = int(item - int64_t(p) * a.g.heads);
-    it.nq = a.nq;
-    it.offset = a.offset;
-    it.q0 = it.head * a.q_h;
-    it.o0 = it.head * a.o_h;
-    it.table_row = a.table;
-    it.kb0 = kb0[p]; it.kb1 = kb1[p]; it.slot = slot[p];
-    return it;
+// Shape of a workgroup's staged round, per element type, padded head dim DP
+// (64 or 128), QT x KG waves and SW, the waves per SIMD its registers are held
+// to (512 registers a lane over the waves of a SIMD). With SW 4 two 8-wave
+// workgroups share a compute unit and hide each other's waits; with fewer the
+// operands of a block are all read before its first MFMA.
+template <int DT, int DP, int QT, int KG, int SW>
+struct CausalShape {
+  static constexpr int ES = elem_bytes<DT>();
+  static constexpr int EC = 16 / ES;     // elements per 16-byte chunk
+  static constexpr int CPR = DP / EC;    // chunks per LDS row
+  static constexpr int KB = 32;          // keys per group and round
+  static constexpr int KI = KG * KB;     // keys per round, a multiple of every page size
+  static constexpr int W = QT * KG;      // waves
+  static constexpr int NT = W * kWave;
+  static constexpr int NC = KI * CPR / NT;     // 16-byte chunks per lane, K and V each
+  static constexpr int RW = kWave / CPR;       // rows one load instruction of a wave fills
+  static constexpr int DT32 = DP / 32;
+  static constexpr int OS = DP + 4;      // row stride of the groups' accumulators in LDS
+  static constexpr int kPlane = KI * DP * ES;  // bytes of a round's K (and V)
+  // Rounds of LDS: one computed, the others in flight.
+  static constexpr int kRing = SW == 4 || KG <= 2 ? 2 : 131072 / (2 * kPlane) < 4 ? 131072 / (2 * kPlane) : 4;
+  static constexpr size_t kStage = size_t(2 * kRing) * kPlane;
+  static constexpr size_t kMerge = KG > 1 ? size_t(KG) * 32 * QT * (OS + 2) * sizeof(float) : 0;
+  static constexpr size_t kLds = kStage > kMerge ? kStage : kMerge;
+  static_assert(NC * NT == KI * CPR && NC >= 1 && kWave % CPR == 0, "a round divides over the workgroup");
+  // Chunk p of key row r lies at chunk kpos / vpos of the row (both their own
+  // inverse). K is read as 16-byte chunks of 32 consecutive rows, V as 4 rows
+  // x 64 bytes (16-bit) or as two rows 4 apart x 128 bytes (fp32).
+  static __device__ __forceinline__ int kpos(int r, int p) { return CPR == 8 ? p ^ ((r >> 1) & 7) : p ^ (r & 15); }
+  static __device__ __forceinline__ int vpos(int r, int p) {
+    if constexpr (DT == kF32) return p ^ (((r >> 2) & 1) << 3);
+    else return CPR == 8 ? p ^ (((r >> 1) & 1) << 2) : p ^ ((r & 3) << 2);
   }
 };
 
-template <int DT, int D, class Items, bool FUSED>
-__global__ __launch_bounds__(kThreads) void prefill_kernel(QueryArgs a, Items items) {
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+template <int DT>
+__device__ __forceinline__ floatx16 mfma32(const u32x4& x, const u32x4& y, const floatx16& c) {
+  if constexpr (DT == kF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(Mfma<kF16>::v8, x),
+                                                  __builtin_bit_cast(Mfma<kF16>::v8, y), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(Mfma<kBF16>::v8, x),
+                                                   __builtin_bit_cast(Mfma<kBF16>::v8, y), c, 0, 0, 0);
+}
+
+// Four keys of one dim: lane t of each 16 lanes passes row t / 4, columns
+// 4 (t % 4) .. + 3 of a 4 x 16 block of 16-bit elements and receives column t.
+__device__ __forceinline__ uint2 read_transposed(const void* p) {
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  const s4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(p));
+  return __builtin_bit_cast(uint2, r);
+}
+
+// acc / l by the output rule (0 for l = 0, NaN for a NaN l) with inv =
+// inverse(l): one multiplication for 16-bit results, corrected to fp32's
+// rounding for fp32 ones.
+__device__ __forceinline__ float inverse(float l) { return l > 0.f ? 1.f / l : (isnan(l) ? NAN : 0.f); }
+template <int DT>
+__device__ __forceinline__ float divided(float acc, float l, float inv) {
+  const float x = acc * inv;
+  if constexpr (DT == kF32) return fmaf(fmaf(-x, l, acc), inv, x);
+  else return x;
+}
+
+// What a staged row reads where there is nothing to read: NaN keys (a missing
+// page: its scores are NaN) and zeros.
+__device__ const uint32_t g_fill[8] = {~0u, ~0u, ~0u, ~0u, 0u, 0u, 0u, 0u};
+
+// Copies 16 bytes per lane from global memory to LDS without passing through
+// registers: lane l's bytes land at lds + 16 l. The compiler does not see the
+// write, nor count it in its own waits: wait_staged() before the barrier that
+// publishes a round.
+__device__ __forceinline__ void stage16(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "m0", "memory");
+}
+__device__ __forceinline__ void stage16(const void* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(base), "v"(offset), "s"(lds)
+               : "m0", "memory");
+}
+__device__ __forceinline__ const char* uniform(const char* p) {
+  const uint64_t x = reinterpret_cast<uintptr_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(x)), hi = __builtin_amdgcn_readfirstlane(uint32_t(x >> 32));
+  return reinterpret_cast<const char*>(uint64_t(hi) << 32 | lo);
+}
+// Waits until at most N of this wave's memory operations are outstanding.
+template <int N>
+__device__ __forceinline__ void wait_staged() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+template <int DT, int DP, int QT, int KG, int SW, class Items, bool FUSED>
+__global__ __launch_bounds__(QT * KG * kWave) __attribute__((amdgpu_waves_per_eu(SW)))
+void causal_kernel(QueryArgs a, Items items) {
   using T = typename Elem<DT>::T;
-  using V8 = typename Mfma<DT>::v8;
-  constexpr int KS = kPfKeys;
-  constexpr int KP = D + 8;     // LDS row of K, padded (elements)
-  constexpr int VP = KS + 8;    // LDS row of V^T, padded
-  constexpr int DT16 = D / 16;  // 16-dim tiles of the output
-  constexpr int DS = D / 32;    // 32-dim steps of q.k
-  constexpr int CPR = D / 8;    // 16-byte chunks per key row
-  constexpr int NC = KS * CPR / kThreads;  // chunks per thread and plane
-  static_assert(NC * kThreads == KS * CPR, "block staging must divide over the workgroup");
+  using S = CausalShape<DT, DP, QT, KG, SW>;
+  constexpr int EC = S::EC, CPR = S::CPR, KB = S::KB, KI = S::KI, NT = S::NT, NC = S::NC, DT32 = S::DT32;
+  constexpr int TQ = 32 * QT;
+  constexpr int QW = DT == kF32 ? DP / 8 : DP / 16;  // 16-byte query registers
   __shared__ const T* s_page[kPfWindowPages];
-  __shared__ __align__(16) T s_k[KS][KP];
-  __shared__ __align__(16) T s_vt[D][VP];
+  __shared__ int s_missing;  // whether a page of a window was missing
+  __shared__ __align__(16) char s_raw[S::kLds];
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)s_raw));
 
   const Geometry& g = a.g;
+  const int dim = g.dim;
+  const int chunks = dim / EC;  // 16-byte chunks per row; the rest of DP is zero
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & (kWave - 1);
-  const int grp = lane >> 4;  // 0..3
-  const int col = lane & 15;  // this lane's query within its wave's 16
+  const int kg = wave / QT, qt = wave - kg * QT;
+  const int grp = lane >> 5;  // 0..1: which half of a block's keys this lane scores
+  const int col = lane & 31;  // this lane's query within its wave's 32
   const T* qp = static_cast<const T*>(a.q);
   T* out = static_cast<T*>(a.out);
   const int win_keys = kPfWindowPages << g.log2_page;
+  // Load n of a wave fills rows row0 + n W RW .. of a round; this lane its row
+  // `sr` further, chunk position `spos`. Pages are at most 32 keys and rounds
+  // start at multiples of 32, so a row's place in its page is fixed.
+  const int sr = wave * S::RW + lane / CPR, spos = lane % CPR;
+  if (tid == 0) s_missing = 0;
 
   const int64_t n_items = items.count(a);
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
-    const PfItem it = items.get(item, a);
-    const int tile = it.tile, head = it.head;
-    const int* table_row = it.table_row;
-    const int nq = it.nq, offset = it.offset, nk = it.offset + it.nq;
+    PfItem it;
+    if (!items.get(item, a, TQ, it)) continue;
+    const int head = it.head;
+    const int nq = it.nq, offset = it.offset;
 
-    // B operand of S^T = K Q^T: dims [32*ds + 8*grp, +8) of query q0 + col.
-    const int q0 = tile * kPfQueries + wave * 16;
+    // B operand of S^T = K Q^T: 16-bit types dims [16 s + 8 grp, + 8) of the
+    // lane's query, fp32 dims [DP / 2 * grp, + DP / 2).
+    const int q0 = it.tile * TQ + qt * 32;
     const int qi = q0 + col;
     const bool q_ok = qi < nq;
-    V8 qv[DS];
-    {
-      const T* row = qp + it.q0 + (q_ok ? qi : 0) * a.q_r;
+    const T* qrow = qp + it.q0 + (q_ok ? qi : 0) * a.q_r;
+    u32x4 qv[QW];
 #pragma unroll
-      for (int ds = 0; ds < DS; ++ds)
-        qv[ds] = __builtin_bit_cast(V8, *global_view(reinterpret_cast<const u32x4*>(row + 32 * ds + 8 * grp)));
+    for (int s = 0; s < QW; ++s) {
+      const int p = DT == kF32 ? CPR / 2 * grp + s : 2 * s + grp;
+      qv[s] = *global_view(reinterpret_cast<const u32x4*>(p < chunks ? qrow + p * EC : reinterpret_cast<const T*>(g_fill + 4)));
     }
     const int qpos = offset + qi;
     const bool wave_live = q0 < nq;
-    const int wave_last = offset + (q0 + 15 < nq ? q0 + 15 : nq - 1);
-    const int tile_q = (tile + 1) * kPfQueries - 1 < nq ? (tile + 1) * kPfQueries - 1 : nq - 1;
-    const int kend = offset + tile_q + 1 < nk ? offset + tile_q + 1 : nk;
+    const int wave_last = offset + (q0 + 31 < nq ? q0 + 31 : nq - 1);
+    const int kend = offset + ((it.tile + 1) * TQ < nq ? (it.tile + 1) * TQ : nq);
 
     float m = -INFINITY, l = 0.f;
-    floatx4 o[DT16];
+    floatx16 o[DT32];
 #pragma unroll
-    for (int dt = 0; dt < DT16; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int d = 0; d < DT32; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
 
-    // Staging of a 64-key block: K row-major, V transposed. Keys past the
-    // window are zero; a missing page is NaN in K (so its score is NaN) and
-    // zero in V (so a query that does not attend it is unaffected). The loads
-    // are issued unconditionally (from this lane's query row when the key has
-    // no page) and the substitution happens at the LDS store, so that no
-    // branch waits for them before the block in between is computed.
-    u32x4 kx[NC], vx[NC];
-    int kstate[NC];  // 0 = loaded, 1 = missing page, 2 = past the window
-    T* wpage[NC];    // page address a staged key of this tile is also written to, or null
-    const T* dummy = qp + it.q0 + (q_ok ? qi : 0) * a.q_r;
-    // FUSED: keys [offset, nk) come from the prompt's own K/V rows, and this
-    // workgroup writes the keys of its own queries, [own0, kend), to the pages.
+    // Staging of a round into LDS half `buf`. Keys past the item's range are
+    // zero; a missing page is NaN in K (so its score is NaN) and zero in V (so
+    // a query that does not attend it is unaffected). FUSED: keys from the
+    // offset on come from the prompt's own K/V rows, and this workgroup writes
+    // the keys of its own queries, [own0, kend), to the pages.
     const T* krows = FUSED ? static_cast<const T*>(a.k) + it.q0 : nullptr;
     const T* vrows = FUSED ? static_cast<const T*>(a.v) + it.q0 : nullptr;
-    const int own0 = offset + tile * kPfQueries;
-    auto stage_load = [&](int k0, int w0, int w1) {
+    const int own0 = offset + it.tile * TQ;
+    const uint64_t row_bytes = uint64_t(a.q_r) * S::ES;
+    const bool short_rows = row_bytes * KI < (uint64_t(1) << 31);
+    auto stage = [&](int k0, int w0, int w1, int buf, bool known, bool plain) {
+      const uint32_t lk = lds0 + buf * 2 * S::kPlane + wave * 1024, lv = lk + S::kPlane;
+      const bool whole = chunks == CPR && plain && k0 + KI <= w1;
+      if (FUSED && whole && k0 >= offset && short_rows) {
+        // a round of the prompt's own rows: one base
+        int row = sr;
+        asm volatile("" : "+v"(row));
+        const char* kb = uniform(reinterpret_cast<const char*>(krows) + uint64_t(uint32_t(k0 - offset)) * row_bytes);
+        const char* vb = uniform(reinterpret_cast<const char*>(vrows) + uint64_t(uint32_t(k0 - offset)) * row_bytes);
 #pragma unroll
-      for (int n = 0; n < NC; ++n) {
-        const int c = tid + n * kThreads;
-        const int kr = c / CPR, part = c - kr * CPR;
-        const int key = k0 + kr;
-        const T* page = key < w1 ? s_page[(key - w0) >> g.log2_page] : nullptr;
-        kstate[n] = key >= w1 ? 2 : (page ? 0 : 1);
-        const T* pk = page ? page + (key & (g.page_size - 1)) * D + part * 8 : nullptr;
-        if constexpr (FUSED) {
-          const bool fresh = key >= offset && key < w1;
-          const T* kp = fresh ? krows + int64_t(key - offset) * a.q_r + part * 8 : (pk ? pk : dummy);
-          const T* vp = fresh ? vrows + int64_t(key - offset) * a.q_r + part * 8 : (pk ? pk + g.kind_stride : dummy);
-          wpage[n] = fresh && pk && key >= own0 ? const_cast<T*>(pk) : nullptr;
-          kx[n] = *global_view(reinterpret_cast<const u32x4*>(kp));
-          vx[n] = *global_view(reinterpret_cast<const u32x4*>(vp));
-        } else {
-          const T* kp = pk ? pk : dummy;
-          const int64_t vstep = pk ? g.kind_stride : 0;
-          kx[n] = *global_view(reinterpret_cast<const u32x4*>(kp));
-          vx[n] = *global_view(reinterpret_cast<const u32x4*>(kp + vstep));
+        for (int n = 0; n < NC; ++n) {
+          const int r = row + n * S::W * S::RW;
+          const uint32_t at = uint32_t(r) * uint32_t(row_bytes);
+          stage16(kb, at + S::kpos(r, spos) * 16, lk + n * S::W * 1024);
+          stage16(vb, at + S::vpos(r, spos) * 16, lv + n * S::W * 1024);
         }
-      }
-    };
-    auto stage_store = [&]() {
+      } else if (whole && (!FUSED || k0 + KI <= offset)) {
+        // a round of present pages
 #pragma unroll
-      for (int n = 0; n < NC; ++n) {
-        const int c = tid + n * kThreads;
-        const int kr = c / CPR, part = c - kr * CPR;
-        const uint32_t kfill = kstate[n] == 1 ? ~0u : 0u;
-        const bool ok = kstate[n] == 0;
-        const u32x4 kk = ok ? kx[n] : u32x4{kfill, kfill, kfill, kfill};
-        *reinterpret_cast<u32x4*>(&s_k[kr][part * 8]) = kk;
-        const uint32_t vw[4] = {ok ? vx[n].x : 0u, ok ? vx[n].y : 0u, ok ? vx[n].z : 0u, ok ? vx[n].w : 0u};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          s_vt[part * 8 + 2 * j][kr] = static_cast<T>(vw[j] & 0xffffu);
-          s_vt[part * 8 + 2 * j + 1][kr] = static_cast<T>(vw[j] >> 16);
+        for (int n = 0; n < NC; ++n) {
+          const int r = sr + n * S::W * S::RW;
+          const T* page = s_page[(k0 + r - w0) >> g.log2_page] + (r & (g.page_size - 1)) * dim;
+          stage16(page + S::kpos(r, spos) * EC, lk + n * S::W * 1024);
+          stage16(page + g.kind_stride + S::vpos(r, spos) * EC, lv + n * S::W * 1024);
         }
-        if constexpr (FUSED) {
-          if (wpage[n]) {  // a key of this tile's own tokens: its page copy
-            *global_view(reinterpret_cast<u32x4*>(wpage[n])) = kx[n];
-            *global_view(reinterpret_cast<u32x4*>(wpage[n] + g.kind_stride)) = vx[n];
+      } else {
+        int row = sr;
+        asm volatile("" : "+v"(row));  // keeps this rare path's terms out of the registers of the loop
+#pragma unroll
+        for (int n = 0; n < NC; ++n) {
+          // a block wholly past the keys is never read
+          if (k0 + ((wave * S::RW + n * S::W * S::RW) & ~(KB - 1)) >= w1) continue;
+          const int r = row + n * S::W * S::RW;
+          const int key = k0 + r;
+          const int pk = S::kpos(r, spos), pv = S::vpos(r, spos);
+          const T* kp = reinterpret_cast<const T*>(g_fill + 4);
+          const T* vp = kp;
+          if (key < w1) {
+            const T* page = known ? s_page[(key - w0) >> g.log2_page] : qp;  // qp: any page, taken as present
+            if (page) {
+              const bool fresh = FUSED && key >= offset;
+              const int64_t at = fresh ? int64_t(uint32_t(key - offset)) * a.q_r : (r & (g.page_size - 1)) * dim;
+              if (pk < chunks) kp = (fresh ? krows : page) + at + pk * EC;
+              if (pv < chunks) vp = (fresh ? vrows : page + g.kind_stride) + at + pv * EC;
+            } else {
+              kp = reinterpret_cast<const T*>(g_fill);
+            }
           }
+          stage16(kp, lk + n * S::W * 1024);
+          stage16(vp, lv + n * S::W * 1024);
         }
       }
     };
     // This item's keys: blocks [kb0, kb1) of [0, kend).
-    const int kstart = it.kb0 * KS;
-    const int kstop = it.kb1 >= (kend + KS - 1) / KS ? kend : it.kb1 * KS;
+    const int kstart = it.kb0 * kPfBlock;
+    const int kstop = int64_t(it.kb1) * kPfBlock < kend ? it.kb1 * kPfBlock : kend;
     for (int w0 = kstart; w0 < kstop; w0 += win_keys) {
       const int w1 = w0 + win_keys < kstop ? w0 + win_keys : kstop;
       const int npg = (w1 - w0 + g.page_size - 1) >> g.log2_page;
-      __syncthreads();
-      for (int j = tid; j < npg; j += kThreads)
-        s_page[j] = page_base<T>(a.slabs, table_row, (w0 >> g.log2_page) + j, g, head);
-      __syncthreads();
-      stage_load(w0, w0, w1);
-      for (int k0 = w0; k0 < w1; k0 += KS) {
-        if (k0 > w0) __syncthreads();  // every wave is done with the previous block
-        stage_store();
-        __syncthreads();
-        // The next block's loads are in flight while this one is computed.
-        if (k0 + KS < w1) stage_load(k0 + KS, w0, w1);
-        if (!wave_live || k0 > wave_last) continue;
-
-        // Scores: lane holds keys k0 + 16*kt + 4*grp + i of query qi.
-        floatx4 sc[4];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-          sc[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ds = 0; ds < DS; ++ds) {
-            const V8 kk = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(&s_k[16 * kt + col][32 * ds + 8 * grp]));
-            sc[kt] = Mfma<DT>::run(kk, qv[ds], sc[kt]);
+      __syncthreads();  // every wave is done with the LDS of the window before
+      // The first round is staged before the window's pages are known when it
+      // holds only the prompt's own rows, and again if one turns out missing.
+      const bool early = FUSED && w0 >= offset;
+      bool plain = true;
+#pragma unroll 1
+      for (int pass = early ? 0 : 1; pass < 2; ++pass) {
+        if (pass == 1) {
+          bool hole = false;
+          for (int j = tid; j < npg; j += NT) {
+            const T* page = page_base<T>(a.slabs, it.table_row, (w0 >> g.log2_page) + j, g, head);
+            s_page[j] = page;
+            hole |= !page;
           }
+          if (hole) s_missing = 1;  // stays set: the careful staging is right for any window
+          __syncthreads();
+          plain = !s_missing;
+          if (!plain) wait_staged<0>();
+        }
+        if (pass == 0 || !early || !plain)
+#pragma unroll 1
+          for (int i = 0; i < S::kRing - 1 && w0 + i * KI < w1; ++i)
+            stage(w0 + i * KI, w0, w1, i, pass == 1, plain);
+      }
+#pragma unroll
+      for (int s = 0; s < QW; ++s) asm volatile("" : "+v"(qv[s]));  // the query has arrived before the loop
+      int buf = 0, ahead = S::kRing - 1;  // the round's LDS, and that of the round staged next
+      for (int k0 = w0; k0 < w1; k0 += KI) {
+        // this wave's part of the round (a round cut short has fewer loads to count)
+        if (k0 + (S::kRing - 1) * KI <= w1) wait_staged<(S::kRing - 2) * 2 * NC>();
+        else wait_staged<0>();
+        __syncthreads();  // everybody's, and the round before is done with
+        if (k0 + (S::kRing - 1) * KI < w1) stage(k0 + (S::kRing - 1) * KI, w0, w1, ahead, true, plain);
+        const T* const s_k = reinterpret_cast<const T*>(s_raw + buf * 2 * S::kPlane);
+        const T* const s_v = reinterpret_cast<const T*>(s_raw + buf * 2 * S::kPlane + S::kPlane);
+        ahead = buf;
+        buf = buf + 1 < S::kRing ? buf + 1 : 0;
+        if (FUSED && k0 + KI > own0) {
+          // keys of this tile's own tokens: their page copies
+          int row = sr;
+          asm volatile("" : "+v"(row));
+#pragma unroll
+          for (int n = 0; n < NC; ++n) {
+            const int r = row + n * S::W * S::RW;
+            const int key = k0 + r;
+            if (key < own0 || key >= w1) continue;
+            T* page = const_cast<T*>(s_page[(key - w0) >> g.log2_page]);
+            if (!page) continue;
+            page += (r & (g.page_size - 1)) * dim;
+            const int pk = S::kpos(r, spos), pv = S::vpos(r, spos);
+            const u32x4 kk = *reinterpret_cast<const u32x4*>(s_k + r * DP + spos * EC);
+            const u32x4 vv = *reinterpret_cast<const u32x4*>(s_v + r * DP + spos * EC);
+            if (pk < chunks) *global_view(reinterpret_cast<u32x4*>(page + pk * EC)) = kk;
+            if (pv < chunks) *global_view(reinterpret_cast<u32x4*>(page + g.kind_stride + pv * EC)) = vv;
+          }
+        }
+        const int base = k0 + kg * KB;  // this wave's block
+        if (!wave_live || base > wave_last || base >= w1) continue;
+
+        // Scores: lane holds keys base + 8 (i / 4) + 4 grp + i % 4 of query qi.
+        floatx16 sc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+        auto read_k = [&](int s) {
+          const int p = DT == kF32 ? CPR / 2 * grp + s : 2 * s + grp;
+          return *reinterpret_cast<const u32x4*>(s_k + (kg * KB + col) * DP + S::kpos(col, p) * EC);
+        };
+        u32x4 kf[SW < 4 ? QW : 1];
+        if constexpr (SW < 4) {
+#pragma unroll
+          for (int s = 0; s < QW; ++s) kf[s] = read_k(s);
+        }
+        // With registers to spare V's operands are read before the scores are worked on.
+        const int t16 = lane & 15;
+        auto read_v = [&](int s, int d) {
+          const int rr = 4 * grp + (t16 >> 2);
+          const int p = 4 * d + ((lane >> 4) & 1) * 2 + ((t16 & 3) >> 1);
+          const T* at = s_v + (kg * KB + 16 * s + rr) * DP + S::vpos(rr, p) * 8 + (t16 & 1) * 4;
+          const uint2 x = read_transposed(at);
+          const uint2 y = read_transposed(at + 8 * DP);
+          return u32x4{x.x, x.y, y.x, y.y};
+        };
+        u32x4 vf[KB / 16][DT32];
+        if constexpr (DT != kF32 && SW < 4) {
+#pragma unroll
+          for (int s = 0; s < KB / 16; ++s)
+#pragma unroll
+            for (int d = 0; d < DT32; ++d) vf[s][d] = read_v(s, d);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (DT == kF32) {
+          // four short chains of sums instead of one of DP / 2
+          floatx16 part[3];
+#pragma unroll
+          for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) part[j][i] = 0.f;
+#pragma unroll
+          for (int s = 0; s < QW; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              floatx16& c = j == 0 ? sc : part[j - 1];
+              c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kf[s][j]), __uint_as_float(qv[s][j]), c, 0, 0, 0);
+            }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sc[i] = (sc[i] + part[0][i]) + (part[1][i] + part[2][i]);
+        } else {
+#pragma unroll
+          for (int s = 0; s < QW; ++s) sc = mfma32<DT>(SW < 4 ? kf[s] : read_k(s), qv[s], sc);
         }
         // Causal / length mask, only for blocks that reach past the wave's
-        // first query or past kend (a wave-uniform test).
-        if (k0 + KS - 1 > offset + q0 || k0 + KS > kend) {
+        // first query or past the item's keys (a wave-uniform test).
+        if (base + KB - 1 > offset + q0 || base + KB > w1) {
+          const int last = min(qpos, w1 - 1) - base - 4 * grp;
 #pragma unroll
-          for (int kt = 0; kt < 4; ++kt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int key = k0 + 16 * kt + 4 * grp + i;
-              if (key > qpos || key >= kend) sc[kt][i] = -INFINITY;
-            }
-          }
+          for (int i = 0; i < 16; ++i)
+            if (8 * (i >> 2) + (i & 3) > last) sc[i] = -INFINITY;
         }
         // Block max of the raw scores (qscale > 0 commutes with the max; NaN
-        // scores are dropped by fmaxf), shared by the four lanes of a query.
-        float bmax = -INFINITY;
+        // scores are dropped by fmaxf), shared by the two lanes of a query.
+        float bmax = sc[0];
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-          bmax = fmaxf(fmaxf(bmax, fmaxf(sc[kt][0], sc[kt][1])), fmaxf(sc[kt][2], sc[kt][3]));
-        bmax = fmaxf(bmax, lane_swap16(bmax));
-        bmax = fmaxf(bmax, lane_swap32(bmax));
-        const float mn = fmaxf(m, bmax * a.qscale);
-        const float alpha = (m == -INFINITY) ? 0.f : fast_exp2(m - mn);
-        const float mref = (mn == -INFINITY) ? 0.f : mn;  // masked scores give exp2(-inf) = 0
-        // B operand of the PV step: k slot j of 32-key step ks holds key
-        // 32*ks + 4*grp + j (j < 4) or 32*ks + 16 + 4*grp + (j - 4). The
-        // denominator stays per lane (this lane's 16 keys) until the end.
-        uint32_t phi[2][4], plo[2][4];
-        float psum = 0.f;
+        for (int i = 1; i < 16; ++i) bmax = fmaxf(bmax, sc[i]);
+        bmax = max_halves(bmax) * a.qscale;
+        if (__any(bmax > m + kRescale)) {  // also a query's first keys, m = -inf
+          const float mn = fmaxf(m, bmax);
+          const float alpha = (m == -INFINITY) ? 0.f : fast_exp2(m - mn);
+          l *= alpha;
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
+          for (int d = 0; d < DT32; ++d)
 #pragma unroll
-          for (int i = 0; i < 4; i += 2) {
-            const float p0 = fast_exp2(fmaf(sc[kt][i], a.qscale, -mref));
-            const float p1 = fast_exp2(fmaf(sc[kt][i + 1], a.qscale, -mref));
-            psum += p0 + p1;
-            const int ks = kt >> 1, w = (kt & 1) * 2 + (i >> 1);
-            float r0, r1;
-            phi[ks][w] = PackP<DT>::pack(p0, p1, r0, r1);
-            plo[ks][w] = PackP<DT>::pack(p0 - r0, p1 - r1, r0, r1);
+            for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
+          m = mn;
+        }
+        const float mref = (m == -INFINITY) ? 0.f : m;  // masked scores give exp2(-inf) = 0
+        float psum[2] = {0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          sc[i] = fast_exp2(fmaf(sc[i], a.qscale, -mref));
+          psum[i & 1] += sc[i];
+        }
+        l += psum[0] + psum[1];  // this lane's keys; the lanes of a query are added at the end
+
+        if constexpr (DT == kF32) {
+          // The block's sums start at zero and are added to the running ones,
+          // so that no chain of sums is longer than a block or the blocks.
+#pragma unroll
+          for (int d = 0; d < DT32; ++d) {
+            floatx16 ob;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) ob[i] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int rr = 8 * (i >> 2) + 4 * grp + (i & 3), dd = 32 * d + col;
+              const float vv = s_v[(kg * KB + rr) * DP + S::vpos(rr, dd >> 2) * 4 + (dd & 3)];
+              ob = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, sc[i], ob, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[d][i] += ob[i];
           }
-        }
-        l = l * alpha + psum;
-        m = mn;
-        V8 pv[2], pl[2];
+        } else {
+          // 16 keys a step: slot j < 4 of a lane holds key 16 s + 4 grp + j,
+          // slot j >= 4 key 16 s + 8 + 4 grp + j - 4, in P as in V^T.
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          pv[ks] = __builtin_bit_cast(V8, u32x4{phi[ks][0], phi[ks][1], phi[ks][2], phi[ks][3]});
-          pl[ks] = __builtin_bit_cast(V8, u32x4{plo[ks][0], plo[ks][1], plo[ks][2], plo[ks][3]});
-        }
+          for (int s = 0; s < KB / 16; ++s) {
+            u32x4 hi, lo;
 #pragma unroll
-        for (int dt = 0; dt < DT16; ++dt) {
+            for (int w = 0; w < 4; ++w) {
+              uint32_t h2, l2;
+              SplitP<DT>::split(sc[8 * s + 2 * w], sc[8 * s + 2 * w + 1], h2, l2);
+              hi[w] = h2;
+              lo[w] = l2;
+            }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[dt][i] *= alpha;
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            // A = V^T rows dt*16 + col, keys in pv's k-slot order.
-            const T* vrow = &s_vt[dt * 16 + col][32 * ks + 4 * grp];
-            const uint2 lo = *reinterpret_cast<const uint2*>(vrow);
-            const uint2 hi = *reinterpret_cast<const uint2*>(vrow + 16);
-            const V8 va = __builtin_bit_cast(V8, u32x4{lo.x, lo.y, hi.x, hi.y});
-            o[dt] = Mfma<DT>::run(va, pv[ks], o[dt]);
-            o[dt] = Mfma<DT>::run(va, pl[ks], o[dt]);
+            for (int d = 0; d < DT32; ++d) {
+              const u32x4 vv = SW < 4 ? vf[s][d] : read_v(s, d);
+              o[d] = mfma32<DT>(vv, hi, o[d]);
+              o[d] = mfma32<DT>(vv, lo, o[d]);
+            }
           }
         }
       }
     }
 
-    // The query's denominator is the sum over its four lanes.
-    l += lane_swap16(l);
-    l += lane_swap32(l);
-    if (q_ok && it.slot >= 0) {
-      // A split of the tile's keys: (max, denominator, accumulators) in
-      // base-2 units for prefill_merge_kernel.
-      float* part = a.partials + ((int64_t(it.slot) * g.heads + head) * kPfQueries + wave * 16 + col) * pf_part_row<D>();
+    // O^T lane layout: dims 32 d + 8 (i / 4) + 4 grp + i % 4 of query qi. A
+    // piece of the tile's keys leaves (accumulators, max, denominator) in
+    // base-2 units for the merge kernels, a whole tile the output rows.
+    l = add_halves(l);
+    float* const part = it.slot >= 0 ? a.partials + (int64_t(it.slot) * g.heads + head) * TQ * pf_part_row<DP>() : nullptr;
+    if constexpr (KG == 1) {
+      const float inv = inverse(l);
 #pragma unroll
-      for (int dt = 0; dt < DT16; ++dt)
-        *reinterpret_cast<float4*>(part + dt * 16 + 4 * grp) = float4{o[dt][0], o[dt][1], o[dt][2], o[dt][3]};
-      if (grp == 0) *reinterpret_cast<float2*>(part + D) = float2{m, l};
-    }
-    // O^T lane layout: dims dt*16 + 4*grp + i of query qi.
-    if (q_ok && it.slot < 0) {
-      T* orow = out + it.o0 + qi * a.o_r;
+      for (int d = 0; d < DT32; ++d)
 #pragma unroll
-      for (int dt = 0; dt < DT16; ++dt) {
-        const T r0 = from_f32<DT>(finalize(o[dt][0], l)), r1 = from_f32<DT>(finalize(o[dt][1], l));
-        const T r2 = from_f32<DT>(finalize(o[dt][2], l)), r3 = from_f32<DT>(finalize(o[dt][3], l));
-        *reinterpret_cast<uint2*>(orow + dt * 16 + 4 * grp) =
-            uint2{uint32_t(r0) | (uint32_t(r1) << 16), uint32_t(r2) | (uint32_t(r3) << 16)};
+        for (int i = 0; i < 16; i += 4) {
+          const int dd = 32 * d + 2 * i + 4 * grp;
+          if (!q_ok) continue;
+          if (part)
+            *reinterpret_cast<float4*>(part + (qt * 32 + col) * pf_part_row<DP>() + dd) =
+                float4{o[d][i], o[d][i + 1], o[d][i + 2], o[d][i + 3]};
+          else if (dd < dim)
+            store4<DT>(out + it.o0 + qi * a.o_r + dd, divided<DT>(o[d][i], l, inv), divided<DT>(o[d][i + 1], l, inv),
+                       divided<DT>(o[d][i + 2], l, inv), divided<DT>(o[d][i + 3], l, inv));
+        }
+      if (part && q_ok && grp == 0)
+        *reinterpret_cast<float2*>(part + (qt * 32 + col) * pf_part_row<DP>() + DP) = float2{m, l};
+    } else {
+      // The groups' states meet in LDS, then every thread merges four dims of
+      // a query over the groups. A group none of whose keys a query attends
+      // holds l = 0; a NaN denominator (missing page) poisons the sum.
+      float* const s_o = reinterpret_cast<float*>(s_raw);
+      float2* const s_ml = reinterpret_cast<float2*>(s_o + KG * TQ * S::OS);
+      __syncthreads();
+      {
+        float* row = s_o + ((kg * TQ) + qt * 32 + col) * S::OS + 4 * grp;
+#pragma unroll
+        for (int d = 0; d < DT32; ++d)
+#pragma unroll
+          for (int i = 0; i < 16; i += 4)
+            *reinterpret_cast<float4*>(row + 32 * d + 2 * i) = float4{o[d][i], o[d][i + 1], o[d][i + 2], o[d][i + 3]};
+        if (grp == 0) s_ml[kg * TQ + qt * 32 + col] = float2{m, l};
+      }
+      __syncthreads();
+      for (int u = tid; u < TQ * DP / 4; u += NT) {
+        const int q = u / (DP / 4), dd = 4 * (u - q * (DP / 4));
+        const int row = it.tile * TQ + q;
+        if (row >= nq) break;
+        float2 ml[KG];
+        float M = -INFINITY, L = 0.f;
+#pragma unroll
+        for (int k = 0; k < KG; ++k) { ml[k] = s_ml[k * TQ + q]; M = fmaxf(M, ml[k].x); }
+        float4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+          const float w = ml[k].x == -INFINITY ? 0.f : fast_exp2(ml[k].x - M);
+          const float4 x = *reinterpret_cast<const float4*>(s_o + (k * TQ + q) * S::OS + dd);
+          L = fmaf(ml[k].y, w, L);
+          acc.x = fmaf(x.x, w, acc.x); acc.y = fmaf(x.y, w, acc.y);
+          acc.z = fmaf(x.z, w, acc.z); acc.w = fmaf(x.w, w, acc.w);
+        }
+        if (part) {
+          float* dst = part + q * pf_part_row<DP>();
+          *reinterpret_cast<float4*>(dst + dd) = acc;
+          if (dd == 0) *reinterpret_cast<float2*>(dst + DP) = float2{M, L};
+        } else if (dd < dim) {
+          const float inv = inverse(L);
+          store4<DT>(out + it.o0 + row * a.o_r + dd, divided<DT>(acc.x, L, inv), divided<DT>(acc.y, L, inv),
+                     divided<DT>(acc.z, L, inv), divided<DT>(acc.w, L, inv));
+        }
       }
     }
   }
 }
 
-// Merge of a split prefill (one request): for each split tile, every query's
-// outputs from its splits' (max, denominator, accumulators) by the log-sum-exp
-// rule, with the finalize rule of the unsplit kernel (a NaN denominator stays
-// NaN, a zero one gives 0). One workgroup per (tile, head), four threads per
-// query, each taking every fourth 16-byte chunk of the row; one online pass
-// over the splits, unrolled so that several splits' loads are in flight.
-struct PrefillMerge {
-  int tiles;
-  unsigned short tile[kSplitPairs], first_slot[kSplitPairs];
-  unsigned char splits[kSplitPairs];
-};
-
-// Key splits of ragged prompts: per split tile, its first output row (in the
-// launch's rows), its valid queries, first partials slot and split count.
-struct RaggedMerge {
-  int tiles;
-  int row0[kSplitPairs];
-  unsigned short nq[kSplitPairs], first_slot[kSplitPairs];
-  unsigned char splits[kSplitPairs];
-};
-
-// Query q of a split tile: log-sum-exp merge of the n partials from slot
-// first_slot on, written to orow (256 threads: 64 queries x 4 column groups).
+// Merge of tiles whose keys were split over workgroups: every query's output
+// from its pieces' (accumulators, max, denominator) by the log-sum-exp rule,
+// with the finalize rule of the unsplit kernel (a NaN denominator stays NaN, a
+// zero one gives 0). One workgroup per (tile, head), four threads per query,
+// each taking every fourth 16-byte chunk of the row; one online pass over the
+// pieces, unrolled so that several pieces' loads are in flight.
 template <int DT, int D>
-__device__ __forceinline__ void merge_query(const QueryArgs& a, int head, int q, int sub, int first_slot, int n,
-                                            typename Elem<DT>::T* orow) {
-  using T = typename Elem<DT>::T;
+__device__ __forceinline__ void merge_query(const QueryArgs& a, int head, int q, int sub, int tq, int first_slot,
+                                            int n, typename Elem<DT>::T* orow) {
   constexpr int R = pf_part_row<D>(), C = D / 16;
-  const float* base = a.partials + ((int64_t(first_slot) * a.g.heads + head) * kPfQueries + q) * R;
-  const int64_t step = int64_t(a.g.heads) * kPfQueries * R;
+  const float* base = a.partials + ((int64_t(first_slot) * a.g.heads + head) * tq + q) * R;
+  const int64_t step = int64_t(a.g.heads) * tq * R;
   float M = -INFINITY, L = 0.f;
   float4 acc[C];
 #pragma unroll
@@ -1718,40 +1939,55 @@ __device__ __forceinline__ void merge_query(const QueryArgs& a, int head, int q,
   }
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    const T r0 = from_f32<DT>(finalize(acc[c].x, L)), r1 = from_f32<DT>(finalize(acc[c].y, L));
-    const T r2 = from_f32<DT>(finalize(acc[c].z, L)), r3 = from_f32<DT>(finalize(acc[c].w, L));
-    *reinterpret_cast<uint2*>(orow + 4 * (sub + 4 * c)) =
-        uint2{uint32_t(r0) | (uint32_t(r1) << 16), uint32_t(r2) | (uint32_t(r3) << 16)};
+    const int dd = 4 * (sub + 4 * c);
+    if (dd < a.g.dim)
+      store4<DT>(orow + dd, finalize(acc[c].x, L), finalize(acc[c].y, L), finalize(acc[c].z, L),
+                 finalize(acc[c].w, L));
   }
 }
 
+// Tiles of a uniform batch: one workgroup per (tile, request, head).
 template <int DT, int D>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(QueryArgs a, PrefillMerge mg) {
+__global__ __launch_bounds__(256) void uniform_merge_kernel(QueryArgs a, UniformItems u, int tq) {
   using T = typename Elem<DT>::T;
-  const int t = int(blockIdx.x / unsigned(a.g.heads));
-  const int head = int(blockIdx.x - unsigned(t) * a.g.heads);
-  if (t >= mg.tiles) return;
-  const int q = threadIdx.x >> 2, sub = threadIdx.x & 3;
-  const int qi = mg.tile[t] * kPfQueries + q;
-  if (qi >= a.nq) return;
-  T* orow = static_cast<T*>(a.out) + head * a.o_h + int64_t(qi) * a.o_r;
-  merge_query<DT, D>(a, head, q, sub, mg.first_slot[t], mg.splits[t], orow);
+  const unsigned bh_count = unsigned(a.batch) * unsigned(a.g.heads);
+  const int tile = int(blockIdx.x / bh_count);
+  const int bh = int(blockIdx.x - unsigned(tile) * bh_count);
+  const int b = bh / a.g.heads, head = bh - b * a.g.heads;
+  const int nb = key_blocks(tile, tq, a.nq, a.offset);
+  if (nb <= u.share) return;  // one piece: its workgroup wrote the output
+  for (int q = threadIdx.x >> 2; q < tq; q += 64) {
+    const int qi = tile * tq + q;
+    if (qi >= a.nq) return;
+    T* orow = static_cast<T*>(a.out) + b * a.o_b + head * a.o_h + int64_t(qi) * a.o_r;
+    merge_query<DT, D>(a, head, q, threadIdx.x & 3, tq, (b * u.tiles + tile) * u.pieces, (nb + u.share - 1) / u.share,
+                       orow);
+  }
 }
+
+// Key splits of ragged prompts: per split tile, its first output row (in the
+// launch's rows), its valid queries, first partials slot and piece count.
+struct RaggedMerge {
+  int tiles;
+  int row0[kRaggedTiles];
+  unsigned short nq[kRaggedTiles], first_slot[kRaggedTiles];
+  unsigned char splits[kRaggedTiles];
+};
 
 // Kernel arguments stay within the 4 KiB kernarg limit.
 static_assert(sizeof(QueryArgs) + sizeof(RaggedItems) <= 4096, "ragged prefill arguments");
 static_assert(sizeof(QueryArgs) + sizeof(RaggedMerge) <= 4096, "ragged merge arguments");
 
 template <int DT, int D>
-__global__ __launch_bounds__(256) void ragged_merge_kernel(QueryArgs a, RaggedMerge mg) {
+__global__ __launch_bounds__(256) void ragged_merge_kernel(QueryArgs a, RaggedMerge mg, int tq) {
   using T = typename Elem<DT>::T;
   const int t = int(blockIdx.x / unsigned(a.g.heads));
   const int head = int(blockIdx.x - unsigned(t) * a.g.heads);
   if (t >= mg.tiles) return;
-  const int q = threadIdx.x >> 2, sub = threadIdx.x & 3;
-  if (q >= mg.nq[t]) return;
-  T* orow = static_cast<T*>(a.out) + head * a.o_h + (int64_t(mg.row0[t]) + q) * a.o_r;
-  merge_query<DT, D>(a, head, q, sub, mg.first_slot[t], mg.splits[t], orow);
+  for (int q = threadIdx.x >> 2; q < mg.nq[t]; q += 64) {
+    T* orow = static_cast<T*>(a.out) + head * a.o_h + (int64_t(mg.row0[t]) + q) * a.o_r;
+    merge_query<DT, D>(a, head, q, threadIdx.x & 3, tq, mg.first_slot[t], mg.splits[t], orow);
+  }
 }
 
 // Multi-token append at a common offset (reference paged_append with
@@ -2161,81 +2397,119 @@ hipError_t launch_append(AppendArgs& a, int dtype) {
   return hipGetLastError();
 }
 
-// Whether launch_query runs the matrix-core prefill kernel: fp16/bf16,
-// head_dim 64/128, 16-byte aligned rows and at least kPfMinQueries queries.
-bool prefill_kernel_takes(const QueryArgs& a, int dtype) {
+// Whether launch_query runs the matrix-core causal kernel: rows of whole
+// 16-byte chunks (head dims 8, 16, .. 128 in fp16/bf16, 4, 8, .. in fp32) at
+// 16-byte aligned addresses and at least kPfMinQueries queries.
+bool causal_kernel_takes(const QueryArgs& a, int dtype) {
   const int d = a.g.dim;
   const int esize = dtype == kF32 ? 4 : 2;
   auto rows16 = [&](int64_t x) { return (x * esize) % 16 == 0; };
-  return (d == 64 || d == 128) && dtype != kF32 && a.nq >= kPfMinQueries && aligned16(a.out) &&
-         aligned16(a.q) && rows16(a.q_b) && rows16(a.q_h) && rows16(a.q_r) && rows16(a.o_b) &&
-         rows16(a.o_h) && rows16(a.o_r);
+  return rows16(d) && a.nq >= kPfMinQueries && aligned16(a.out) && aligned16(a.q) && rows16(a.q_b) &&
+         rows16(a.q_h) && rows16(a.q_r) && rows16(a.o_b) && rows16(a.o_h) && rows16(a.o_r);
 }
 
-// Launches that took the key-split prefill path (a diagnostic for tests).
+// Launches that split long prompts' keys (a diagnostic for tests).
 std::atomic<long long> g_key_split_launches{0};
 
-// Key-split prefill of one request whose query tiles give at most one
-// workgroup per compute unit and whose last tile walks many key blocks: each tile's keys are cut
-// into splits of B blocks (B chosen for about two workgroups per compute
-// unit), every split a workgroup, the splits then merged. Returns
-// hipErrorNotSupported when the shape is better served unsplit.
-hipError_t launch_split_prefill(QueryArgs& a, int dtype) {
-  const int h = a.g.heads, d = a.g.dim;
-  const int tiles = (a.nq + kPfQueries - 1) / kPfQueries;
-  const int cus = device_compute_units();
-  auto blocks_of = [&](int t) {
-    const int64_t last = int64_t(a.offset) + std::min(int64_t(t + 1) * kPfQueries, int64_t(a.nq));
-    return int((std::min<int64_t>(last, a.nk) + kPfKeys - 1) / kPfKeys);
-  };
-  if (a.batch != 1 || cus < 1 || int64_t(tiles) * h > cus || blocks_of(tiles - 1) < 6)
-    return hipErrorNotSupported;
-  int64_t total = 0;
-  for (int t = 0; t < tiles; ++t) total += blocks_of(t);
-  const int B = std::max<int>(2, int((total * h + 2 * cus - 1) / (2 * cus)));
-  SplitItems it{};
-  PrefillMerge mg{};
-  int pairs = 0, slots = 0;
-  for (int t = tiles - 1; t >= 0; --t) {  // heaviest tiles first
-    const int nb = blocks_of(t), n = (nb + B - 1) / B;
-    if (pairs + n > kSplitPairs || n > 255 || nb > 65535) return hipErrorNotSupported;
-    if (n > 1) {
-      mg.tile[mg.tiles] = static_cast<unsigned short>(t);
-      mg.first_slot[mg.tiles] = static_cast<unsigned short>(slots);
-      mg.splits[mg.tiles] = static_cast<unsigned char>(n);
-      ++mg.tiles;
-    }
-    for (int s = 0; s < n; ++s) {
-      it.tile[pairs] = static_cast<unsigned short>(t);
-      it.kb0[pairs] = static_cast<unsigned short>(s * B);
-      it.kb1[pairs] = static_cast<unsigned short>(std::min(nb, (s + 1) * B));
-      it.slot[pairs] = static_cast<short>(n > 1 ? slots++ : -1);
-      ++pairs;
-    }
+// Workgroup shapes of a causal launch (QT x KG waves, SW): queries per tile
+// and how many ways the tile's keys are split inside the workgroup.
+enum CausalConfig : int {
+  kTiny,    // 64 queries, unsplit: two waves and rounds of 32 keys, for prompts of one key block
+  kShort,   // 64 queries, 2 ways: four waves and rounds of 64 keys, for two key blocks
+  kNarrow,  // 32 queries, up to 8 ways
+  kDeep,    // 64 queries, 4 ways
+  kDense,   // 64 queries, 4 ways, two workgroups per compute unit (16-bit types, head dims to 64)
+  kWide     // 128 queries, 2 ways, two workgroups per compute unit likewise
+};
+int config_queries(int config) { return config == kNarrow ? 32 : config == kWide ? 128 : 64; }
+
+// How a causal launch runs: its shape, and with share > 0 the blocks of
+// kPfBlock keys after which a tile's keys go to another workgroup.
+struct CausalPlan {
+  int config, share;
+};
+
+// tiles32/64/128: workgroups (tiles x heads, over all prompts) for tiles of
+// that many queries; blocks: key blocks of the longest tile; row_bytes: a K
+// row in LDS. Where the lines lie (MI355X, 256 compute units, us per call):
+// * kTiny and kShort for prompts of one and two key blocks, which end before
+//   wider workgroups have met: 8 x 100 tokens x 25 heads fp16 9.3 kShort
+//   against 11.5 kDense.
+// * kNarrow while its workgroups take one round of the compute units (an
+//   eighth more still end with the long tiles): 300 tokens x 12 heads bf16 8.0
+//   against 8.8 kDeep, 700 x 12 fp32 (264 workgroups) 25.8 against 33.1; but
+//   1000 x 16 bf16 (512) 17.5 against 15.2 kDeep.
+// * kDeep while 64-query tiles take one round; then kDense, whose second
+//   workgroup per compute unit covers for the first: 1000 x 25 bf16 18.9
+//   against 21.5 kDeep and 24.8 kWide.
+// * kWide from one and a half rounds of 128-query tiles on, when what a tile
+//   spends outside its key loop counts: 8 x 512 tokens x 25 heads 33.1
+//   against 42.9 kDense; below it kDense (2048 at offset 2048 x 16: 60 against 76).
+// * Splitting over workgroups costs a merge launch (about 5 us): only when
+//   narrow tiles leave half the compute units idle and the longest walks at
+//   least 8 rounds, in pieces of at least 3 (40 tokens at offset 4000 x 12
+//   heads bf16: 15.5 against 26.9).
+CausalPlan causal_plan(int64_t tiles32, int64_t tiles64, int64_t tiles128, int blocks, int row_bytes) {
+  const int64_t cus = std::max(1, device_compute_units());
+  CausalPlan plan{};
+  plan.config = blocks == 1 ? kTiny : blocks == 2 ? kShort : 8 * tiles32 <= 9 * cus ? kNarrow : tiles64 <= cus ? kDeep : 2 * tiles128 < 3 * cus ? kDense : kWide;
+  const int round = std::max(1, 4 * 128 / row_bytes);  // blocks a narrow workgroup takes per round
+  if (plan.config == kNarrow && 2 * tiles32 <= cus && blocks >= 8 * round) {
+    const int64_t pieces = std::min<int64_t>(std::min<int64_t>(cus / tiles32, 64), blocks / (3 * round));
+    plan.share = int((blocks + pieces - 1) / pieces);
   }
-  if (mg.tiles == 0) return hipErrorNotSupported;
-  it.pairs = pairs;
-  void* ws = nullptr;
-  // Without room for the partials the prompt runs unsplit.
-  if (library_workspace(size_t(slots) * h * kPfQueries * (d + 4) * sizeof(float), &ws) != hipSuccess)
-    return hipErrorNotSupported;
-  a.partials = static_cast<float*>(ws);
-  const int blocks = grid_for(int64_t(pairs) * h);
-#define MT_SPLIT(DT, D)                                                                        \
-  if (a.k) prefill_kernel<DT, D, SplitItems, true><<<blocks, kThreads>>>(a, it);              \
-  else prefill_kernel<DT, D, SplitItems, false><<<blocks, kThreads>>>(a, it);                 \
-  prefill_merge_kernel<DT, D><<<unsigned(mg.tiles * h), 256>>>(a, mg);
-  if (dtype == kF16) {
-    if (d == 64) { MT_SPLIT(kF16, 64) }
-    else { MT_SPLIT(kF16, 128) }
+  return plan;
+}
+
+// Counts a launch that shortened its longest tiles by splitting their keys
+// over wave groups or workgroups: tiles of at least 6 blocks whose prompts
+// alone would not have kept the compute units busy.
+void count_key_split(bool idle, int blocks) {
+  if (idle && blocks >= 6) g_key_split_launches.fetch_add(1, std::memory_order_relaxed);
+}
+
+template <int DT, int DP, class Items, bool FUSED>
+void launch_causal_t(int config, int blocks, const QueryArgs& a, const Items& items) {
+  constexpr int CPR = DP * elem_bytes<DT>() / 16;
+  constexpr int SW = CPR == 32 ? 1 : 2;              // waves per SIMD the operands leave room for
+  constexpr int NK = CPR == 8 ? 8 : CPR == 16 ? 4 : 2;  // ways a narrow tile's keys are split
+  constexpr int DK = CPR == 32 ? 2 : 4;
+  if (config == kTiny) {
+    causal_kernel<DT, DP, 2, 1, SW, Items, FUSED><<<blocks, 2 * kWave>>>(a, items);
+  } else if (config == kShort) {
+    causal_kernel<DT, DP, 2, 2, CPR == 8 ? 3 : SW, Items, FUSED><<<blocks, 4 * kWave>>>(a, items);
+  } else if (config == kNarrow) {
+    causal_kernel<DT, DP, 1, NK, CPR == 8 ? 2 : 1, Items, FUSED><<<blocks, NK * kWave>>>(a, items);
+  } else if constexpr (CPR == 8) {
+    if (config == kDeep) causal_kernel<DT, DP, 2, 4, 2, Items, FUSED><<<blocks, 8 * kWave>>>(a, items);
+    else if (config == kDense) causal_kernel<DT, DP, 2, 4, 4, Items, FUSED><<<blocks, 8 * kWave>>>(a, items);
+    else causal_kernel<DT, DP, 4, 2, 4, Items, FUSED><<<blocks, 8 * kWave>>>(a, items);
+  } else if (config == kWide) {
+    causal_kernel<DT, DP, 4, DK / 2, SW, Items, FUSED><<<blocks, 2 * DK * kWave>>>(a, items);
   } else {
-    if (d == 64) { MT_SPLIT(kBF16, 64) }
-    else { MT_SPLIT(kBF16, 128) }
+    causal_kernel<DT, DP, 2, DK, SW, Items, FUSED><<<blocks, 2 * DK * kWave>>>(a, items);
   }
-#undef MT_SPLIT
-  const hipError_t e = hipGetLastError();
-  if (e == hipSuccess) g_key_split_launches.fetch_add(1, std::memory_order_relaxed);
-  return e;
+}
+template <int DT, class Items>
+void launch_causal_dt(int config, int blocks, const QueryArgs& a, const Items& items) {
+  const bool small = a.g.dim <= 64;
+  if constexpr (std::is_same<Items, RaggedItems>::value) {
+    if (small) launch_causal_t<DT, 64, Items, true>(config, blocks, a, items);
+    else launch_causal_t<DT, 128, Items, true>(config, blocks, a, items);
+  } else if (a.k) {
+    if (small) launch_causal_t<DT, 64, Items, true>(config, blocks, a, items);
+    else launch_causal_t<DT, 128, Items, true>(config, blocks, a, items);
+  } else {
+    if (small) launch_causal_t<DT, 64, Items, false>(config, blocks, a, items);
+    else launch_causal_t<DT, 128, Items, false>(config, blocks, a, items);
+  }
+}
+template <class Items>
+void launch_causal(int config, int dtype, int64_t items_count, const QueryArgs& a, const Items& items) {
+  const int blocks = grid_for(items_count);
+  if (dtype == kF32) launch_causal_dt<kF32>(config, blocks, a, items);
+  else if (dtype == kF16) launch_causal_dt<kF16>(config, blocks, a, items);
+  else launch_causal_dt<kBF16>(config, blocks, a, items);
 }
 
 // Causal attention launch for any q/out strides: the matrix-core prefill
@@ -2249,22 +2523,38 @@ hipError_t launch_query(QueryArgs& a, int dtype) {
                    rows16(a.q_h) && rows16(a.q_r) && rows16(a.o_b) && rows16(a.o_h) && rows16(a.o_r);
   a.qscale = (1.0f / std::sqrt(float(d))) * kLog2e;
   const int h = a.g.heads;
-  if (prefill_kernel_takes(a, dtype)) {
-    const hipError_t split = launch_split_prefill(a, dtype);
-    if (split != hipErrorNotSupported) return split;
-    a.items = int64_t(a.batch) * h * ((a.nq + kPfQueries - 1) / kPfQueries);
-    const int blocks = grid_for(a.items);
-#define MT_PREFILL(DT, D)                                                                   \
-  if (a.k) prefill_kernel<DT, D, UniformItems, true><<<blocks, kThreads>>>(a, UniformItems{});   \
-  else prefill_kernel<DT, D, UniformItems, false><<<blocks, kThreads>>>(a, UniformItems{});
-    if (dtype == kF16) {
-      if (d == 64) { MT_PREFILL(kF16, 64) }
-      else { MT_PREFILL(kF16, 128) }
-    } else {
-      if (d == 64) { MT_PREFILL(kBF16, 64) }
-      else { MT_PREFILL(kBF16, 128) }
+  if (causal_kernel_takes(a, dtype)) {
+    const int64_t bh = int64_t(a.batch) * h;
+    auto tiles = [&](int tq) { return (a.nq + tq - 1) / tq; };
+    const int most = key_blocks(tiles(64) - 1, 64, a.nq, a.offset);
+    const CausalPlan plan = causal_plan(bh * tiles(32), bh * tiles(64), bh * tiles(128), most,
+                                         (d <= 64 ? 64 : 128) * esize);
+    const int tq = config_queries(plan.config);
+    UniformItems items{tiles(tq), 1, 0};
+    if (plan.share > 0) {
+      const int pieces = (most + plan.share - 1) / plan.share;
+      void* ws = nullptr;
+      // Without room for the partials the launch runs unsplit.
+      if (pieces > 1 && library_workspace(size_t(bh) * items.tiles * pieces * tq * (d <= 64 ? 68 : 132) * sizeof(float),
+                                          &ws) == hipSuccess) {
+        items.pieces = pieces;
+        items.share = plan.share;
+        a.partials = static_cast<float*>(ws);
+      }
     }
-#undef MT_PREFILL
+    a.items = bh * items.tiles * items.pieces;
+    launch_causal(plan.config, dtype, a.items, a, items);
+    if (items.pieces > 1) {
+      const int blocks = grid_for(bh * items.tiles);
+#define MT_MERGE(DT)                                                              \
+  if (d <= 64) uniform_merge_kernel<DT, 64><<<blocks, 256>>>(a, items, tq);       \
+  else uniform_merge_kernel<DT, 128><<<blocks, 256>>>(a, items, tq);
+      if (dtype == kF32) { MT_MERGE(kF32) }
+      else if (dtype == kF16) { MT_MERGE(kF16) }
+      else { MT_MERGE(kBF16) }
+#undef MT_MERGE
+    }
+    count_key_split(a.batch == 1 && bh * tiles(64) <= device_compute_units(), most);
     return hipGetLastError();
   }
   if (a.k) return hipErrorInvalidValue;
@@ -2339,7 +2629,7 @@ int mt_paged_prefill(void* out, const void* q, const void* k, const void* v, con
   a.g = make_geometry(h, d, page_size, pages_per_slab, num_slabs, columns, layer);
   a.q_b = int64_t(n) * qkv_stride; a.q_h = d; a.q_r = qkv_stride;
   a.o_b = int64_t(n) * out_stride; a.o_h = d; a.o_r = out_stride;
-  if (prefill_kernel_takes(a, dtype) && aligned16(k) && aligned16(v)) {
+  if (causal_kernel_takes(a, dtype) && aligned16(k) && aligned16(v)) {
     // The prefill kernel reads the new keys from k/v and writes them to
     // their pages itself: no separate append.
     a.k = k; a.v = v;
@@ -2377,8 +2667,8 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
   if (total * qkv_stride > INT32_MAX || total * out_stride > INT32_MAX) return hipErrorInvalidValue;
   const size_t e = dtype == kF32 ? 4 : 2;
   auto rows16 = [&](int64_t x) { return (x * int64_t(e)) % 16 == 0; };
-  const bool mfma = dtype != kF32 && (d == 64 || d == 128) && aligned16(out) && aligned16(q) &&
-                    aligned16(k) && aligned16(v) && rows16(qkv_stride) && rows16(out_stride) && rows16(d);
+  const bool mfma = aligned16(out) && aligned16(q) && aligned16(k) && aligned16(v) && rows16(qkv_stride) &&
+                    rows16(out_stride) && rows16(d);
   if (!mfma) {
     // Shapes the matrix-core kernel does not take: one call per prompt.
     int64_t first = 0;
@@ -2400,16 +2690,21 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
   int64_t row0 = 0;
   while (r0 < requests) {
     RaggedItems it{};
-    int r1 = r0, pairs = 0;
+    int r1 = r0;
     int64_t rows = 0;
-    while (r1 < requests && r1 - r0 < kRaggedPrompts &&
-           pairs + (tokens[r1] + kPfQueries - 1) / kPfQueries <= kRaggedTiles) {
+    int most = 0;  // key blocks of the longest tile
+    int64_t tiles32 = 0, tiles64 = 0, tiles128 = 0, total_blocks = 0;
+    while (r1 < requests && r1 - r0 < kRaggedPrompts && tiles64 + (tokens[r1] + 63) / 64 <= kRaggedTiles) {
       const int p = r1 - r0;
       it.first_row[p] = int(rows);
       it.n[p] = tokens[r1];
       it.offset[p] = offsets[r1];
       it.table[p] = tables[r1];
-      pairs += (tokens[r1] + kPfQueries - 1) / kPfQueries;
+      most = std::max(most, key_blocks((tokens[r1] - 1) / 64, 64, tokens[r1], offsets[r1]));
+      for (int t = 0; t * 64 < tokens[r1]; ++t) total_blocks += key_blocks(t, 64, tokens[r1], offsets[r1]);
+      tiles32 += (tokens[r1] + 31) / 32;
+      tiles64 += (tokens[r1] + 63) / 64;
+      tiles128 += (tokens[r1] + 127) / 128;
       rows += tokens[r1];
       ++r1;
     }
@@ -2427,76 +2722,55 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
       continue;
     }
     it.prompts = r1 - r0;
-    it.pairs = pairs;
-    // (prompt, tile) pairs, the tiles that attend the most keys first.
-    std::vector<std::pair<int, int>> order;
-    for (int p = 0; p < it.prompts; ++p)
-      for (int t = 0; t * kPfQueries < it.n[p]; ++t) order.push_back({p, t});
-    std::stable_sort(order.begin(), order.end(), [&](const std::pair<int, int>& x, const std::pair<int, int>& y) {
-      auto keys = [&](const std::pair<int, int>& z) {
-        const int last = (z.second + 1) * kPfQueries < it.n[z.first] ? (z.second + 1) * kPfQueries : it.n[z.first];
-        return it.offset[z.first] + last;
-      };
-      return keys(x) > keys(y);
-    });
-    // Key splits: a tile whose keys span more blocks than its share of the
-    // launch (all pairs' key blocks times the heads over two workgroups per
-    // compute unit, at least 2) is cut into pieces of at most that many
-    // blocks, merged afterwards by ragged_merge_kernel. Only when the longest
-    // tile has at least 6 blocks, as for one prompt (launch_split_prefill).
-    auto blocks_of = [&](const std::pair<int, int>& z) {
-      const int last = (z.second + 1) * kPfQueries < it.n[z.first] ? (z.second + 1) * kPfQueries : it.n[z.first];
-      return (it.offset[z.first] + last + kPfKeys - 1) / kPfKeys;
-    };
-    int64_t total_blocks = 0;
-    int max_blocks = 0;
-    for (const auto& z : order) {
-      total_blocks += blocks_of(z);
-      max_blocks = std::max(max_blocks, blocks_of(z));
-    }
-    const int cus = device_compute_units();
-    const int share = MT_RAGGED_SHARE * std::max(cus, 1);
-    int B = std::max<int>(2, int((total_blocks * h + share - 1) / share));
-    auto pieces = [&](int B) {
-      int64_t c = 0;
-      for (const auto& z : order) c += (blocks_of(z) + B - 1) / B;
-      return c;
-    };
-    while (pieces(B) > kRaggedTiles) ++B;
-    bool split = MT_RAGGED_KEY_SPLIT && cus > 0 && max_blocks >= 6 && max_blocks > B && max_blocks <= 65535;
-    struct Piece { int p, t, kb0, kb1, slot; };
-    std::vector<Piece> list;
+    // (narrow tiles only where the launch can list them)
+    const CausalPlan plan = causal_plan(tiles32 <= kRaggedTiles ? tiles32 * h : INT64_MAX / 16, tiles64 * h,
+                                        tiles128 * h, most, (d <= 64 ? 64 : 128) * int(e));
+    const int tq = config_queries(plan.config);
+    // (prompt, tile) pairs and their key blocks, the longest first; with a
+    // share, cut into pieces of at most that many blocks as far as the
+    // launch describes them.
+    struct Piece { int p, t, kb0, kb1, slot, at; };
+    Piece list[kRaggedTiles];
     RaggedMerge mg{};
-    int slots = 0;
-    if (split) {
-      for (const auto& z : order) {
-        const int nb = blocks_of(z), n = (nb + B - 1) / B;
-        if (n > 1) {
-          mg.row0[mg.tiles] = it.first_row[z.first] + z.second * kPfQueries;
-          mg.nq[mg.tiles] = static_cast<unsigned short>(std::min(kPfQueries, it.n[z.first] - z.second * kPfQueries));
-          mg.first_slot[mg.tiles] = static_cast<unsigned short>(slots);
-          mg.splits[mg.tiles] = static_cast<unsigned char>(n);
-          ++mg.tiles;
+    int share = plan.share, pairs = 0, slots = 0;
+    auto cut = [&](bool write) {
+      int count = 0;
+      for (int p = 0; p < it.prompts; ++p)
+        for (int t = 0; t * tq < it.n[p]; ++t) {
+          const int nb = key_blocks(t, tq, it.n[p], it.offset[p]);
+          const int n = share > 0 ? (nb + share - 1) / share : 1;
+          if (write) {
+            if (n > 1) {
+              mg.row0[mg.tiles] = it.first_row[p] + t * tq;
+              mg.nq[mg.tiles] = static_cast<unsigned short>(std::min(tq, it.n[p] - t * tq));
+              mg.first_slot[mg.tiles] = static_cast<unsigned short>(slots);
+              mg.splits[mg.tiles] = static_cast<unsigned char>(n);
+              ++mg.tiles;
+            }
+            for (int j = 0; j < n; ++j)
+              list[count + j] = {p, t, j * share, n > 1 ? std::min(nb, (j + 1) * share) : nb, n > 1 ? slots++ : -1, count + j};
+          }
+          count += n;
         }
-        for (int j = 0; j < n; ++j)
-          list.push_back({z.first, z.second, j * B, std::min(nb, (j + 1) * B), n > 1 ? slots++ : -1});
-      }
-      // Heaviest pieces first.
-      std::stable_sort(list.begin(), list.end(),
-                       [](const Piece& x, const Piece& y) { return x.kb1 - x.kb0 > y.kb1 - y.kb0; });
-    } else {
-      for (const auto& z : order) list.push_back({z.first, z.second, 0, blocks_of(z), -1});
-    }
+      return count;
+    };
+    while (share > 0 && cut(false) > kRaggedTiles) ++share;
     void* ws = nullptr;
-    // Without room for the partials the launch runs unsplit.
-    if (split && (mg.tiles > kSplitPairs || slots > 32767 ||
-                  library_workspace(size_t(slots) * h * kPfQueries * (d + 4) * sizeof(float), &ws) != hipSuccess)) {
-      split = false;
-      list.clear();
-      mg = RaggedMerge{};
-      for (const auto& z : order) list.push_back({z.first, z.second, 0, blocks_of(z), -1});
+    if (share > 0) {
+      // Without room for the partials the launch runs unsplit.
+      pairs = cut(true);
+      if (most > 65535 ||
+          (slots && library_workspace(size_t(slots) * h * tq * (d <= 64 ? 68 : 132) * sizeof(float), &ws) != hipSuccess)) {
+        share = slots = 0;
+        mg = RaggedMerge{};
+      }
     }
-    pairs = int(list.size());
+    if (share == 0) pairs = cut(true);
+    std::sort(list, list + pairs, [](const Piece& x, const Piece& y) {
+      const int nx = x.kb1 - x.kb0, ny = y.kb1 - y.kb0;
+      return nx != ny ? nx > ny : x.at < y.at;
+    });
+    const bool split = slots > 0;
     it.pairs = pairs;
     for (int i = 0; i < pairs; ++i) {
       it.pair_prompt[i] = static_cast<unsigned char>(list[i].p);
@@ -2517,27 +2791,21 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
     a.q_h = d; a.q_r = qkv_stride;
     a.o_h = d; a.o_r = out_stride;
     a.partials = static_cast<float*>(ws);
-    const int blocks = grid_for(int64_t(pairs) * h);
-    if (dtype == kF16) {
-      if (d == 64) prefill_kernel<kF16, 64, RaggedItems, true><<<blocks, kThreads>>>(a, it);
-      else prefill_kernel<kF16, 128, RaggedItems, true><<<blocks, kThreads>>>(a, it);
-    } else {
-      if (d == 64) prefill_kernel<kBF16, 64, RaggedItems, true><<<blocks, kThreads>>>(a, it);
-      else prefill_kernel<kBF16, 128, RaggedItems, true><<<blocks, kThreads>>>(a, it);
-    }
+    launch_causal(plan.config, dtype, int64_t(pairs) * h, a, it);
     if (split) {
       const unsigned mblocks = unsigned(mg.tiles * h);
-      if (dtype == kF16) {
-        if (d == 64) ragged_merge_kernel<kF16, 64><<<mblocks, 256>>>(a, mg);
-        else ragged_merge_kernel<kF16, 128><<<mblocks, 256>>>(a, mg);
-      } else {
-        if (d == 64) ragged_merge_kernel<kBF16, 64><<<mblocks, 256>>>(a, mg);
-        else ragged_merge_kernel<kBF16, 128><<<mblocks, 256>>>(a, mg);
-      }
+#define MT_MERGE(DT)                                                            \
+  if (d <= 64) ragged_merge_kernel<DT, 64><<<mblocks, 256>>>(a, mg, tq);        \
+  else ragged_merge_kernel<DT, 128><<<mblocks, 256>>>(a, mg, tq);
+      if (dtype == kF32) { MT_MERGE(kF32) }
+      else if (dtype == kF16) { MT_MERGE(kF16) }
+      else { MT_MERGE(kBF16) }
+#undef MT_MERGE
     }
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    if (split) g_key_split_launches.fetch_add(1, std::memory_order_relaxed);
+    // the longest tile against its share of the launch over two workgroups per compute unit
+    count_key_split(int64_t(most) * 2 * std::max(1, device_compute_units()) > total_blocks * h, most);
     r0 = r1;
     row0 += rows;
   }

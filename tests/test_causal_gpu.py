@@ -1,0 +1,47 @@
+"""GPU parity of the matrix-core causal attention at the edges of its tiles and
+of its dispatch, against the float64 oracle: head dims that do not fill the
+kernel's 64 or 128 columns, fp32, query counts around the 32-, 64- and
+128-query tiles, every workgroup shape and keys split over workgroups.
+Tolerances are in tests/tolerances.py."""
+import pytest
+
+from test_prefill_gpu import prefill_case, run_prefill, run_fused_single, run_ragged
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('dtype,dim', [('float32', 64), ('float32', 128), ('float32', 20), ('float16', 32),
+                                       ('bfloat16', 80), ('float16', 128), ('bfloat16', 8)])
+@pytest.mark.parametrize('nq,offset', [(2, 0), (31, 33), (33, 0), (65, 31), (129, 250)])
+def test_causal_tile_edges(dtype, dim, nq, offset):
+    case = prefill_case(200 + dim + nq, batch=2, heads=2, dim=dim, page_size=16, nk=offset + nq, dtype=dtype,
+                        layers=2, layer=1)
+    run_prefill(case, nq, offset + nq, offset, seed=nq)
+    one = prefill_case(300 + dim + nq, batch=1, heads=2, dim=dim, page_size=8, nk=offset + nq, dtype=dtype)
+    run_fused_single(one, nq, offset, seed=nq)
+
+
+# (batch, heads, queries): 64-query tiles in one round of the compute units,
+# two 64-query workgroups per compute unit, 128-query tiles
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('batch,heads,nq,offset', [(3, 20, 200, 5), (3, 40, 200, 5), (5, 60, 140, 5)])
+def test_causal_workgroup_shapes(dtype, batch, heads, nq, offset):
+    case = prefill_case(400 + nq, batch=batch, heads=heads, dim=64, page_size=16, nk=offset + nq, dtype=dtype)
+    run_prefill(case, nq, offset + nq, offset, seed=heads)
+
+
+@pytest.mark.parametrize('dtype,dim', [('float32', 64), ('bfloat16', 64), ('float16', 80)])
+@pytest.mark.parametrize('nq,offset', [(3, 4090), (40, 2500)])
+def test_causal_keys_split_over_workgroups(dtype, dim, nq, offset):
+    # few tiles, many rounds of keys; a hole is NaN for every query through the merge
+    case = prefill_case(500 + nq, batch=1, heads=2, dim=dim, page_size=8, nk=offset + nq, dtype=dtype,
+                        pages_per_slab=16)
+    run_prefill(case, nq, offset + nq, offset, seed=nq)
+    run_fused_single(case, nq, offset, seed=nq)
+    case.table[0, 100] = -1
+    run_prefill(case, nq, offset + nq, offset, seed=nq)
+
+
+@pytest.mark.parametrize('dtype,dim', [('float32', 64), ('bfloat16', 80)])
+def test_causal_ragged_splits_over_workgroups(dtype, dim):
+    run_ragged(dtype, dim, [1, 33, 20], [2600, 17, 2100], h=2, seed=dim)
