@@ -40,13 +40,16 @@ int mt_paged_attention(void* out, const void* q, const uint64_t* slabs, const in
 /* Ragged batched decode: q/k/v/out [b, h, 1, d]; offsets[b] (device) are the
  * committed lengths. Appends k/v at position offsets[i] of request i, then
  * attends its offsets[i] + 1 keys. One fused append + attention launch, plus
- * a split-reduction launch when the table is longer than one context split
- * (1024 tokens). Rows are visited longest first, in the order
- * mt_paged_decode_split takes from a host work list, ranked on the device:
- * when no row can split and b <= 256 every workgroup ranks the rows by
- * offsets[] itself; otherwise, up to 2048 rows, a one-workgroup launch
+ * a split-reduction launch when the table is longer than 1024 tokens (the
+ * split length is then 1024 tokens, longer or shorter: longer for tables that
+ * would need more than 8 splits, shorter where b * h rows alone leave compute
+ * units idle). A batch of more rows than the compute units hold is visited
+ * longest first, in the order mt_paged_decode_split takes from a host work
+ * list, ranked on the device: when no row can split and b <= 256 every
+ * workgroup ranks the rows by offsets[] itself; otherwise, up to 2048 rows and
+ * from 16 workgroups per compute unit on, a one-workgroup launch
  * (mt_paged_decode_order) writes the work list first and one residency
- * round of workgroups strides over it. Larger batches are visited in batch
+ * round of workgroups strides over it. Other batches are visited in batch
  * order. The split partials and that list live in a library-owned
  * device workspace, one per (host thread, device) -- so calls from several
  * host threads, each on its own default stream, never share one -- kept
@@ -71,9 +74,9 @@ int mt_paged_decode_batch(void* out, const void* q, const void* k, const void* v
  * MT_PAGED_NOALLOC_SCRATCH_BYTES instead of a workspace that may grow, and so
  * does the device-built visiting order. It returns 1 (invalid value) before
  * any launch when the partials, b * h * n * (d' + 2) * 4 bytes rounded up to
- * 256 (n = ceil(columns * page_size / split), d' = 64 for 16-byte-aligned
+ * 256 (n = ceil(columns * page_size / split) for the split length above, d' = 64 for 16-byte-aligned
  * operands at d = 64, else 128; none when n = 1), plus the order,
- * (2 + (2 n + 1) b) * 4 bytes (none when n = 1 and b <= 256), exceed that
+ * (2 + (2 n + 1) b) * 4 bytes (none when no order is built), exceed that
  * size. Calls on one device share the array: calls
  * that overlap (different streams) race; calls in stream order do not. The
  * first call on a device looks the array's device address up

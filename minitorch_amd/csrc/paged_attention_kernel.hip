@@ -273,10 +273,25 @@ __device__ __forceinline__ float group_sum(float x) {
   return x;
 }
 
+// How a decode reads rows: element by element, masked to the head dim; in
+// 16-byte loads when the head dim is the kernel's (64 or 128); in 16-byte
+// loads masked to a smaller head dim of whole 16-byte chunks (80 of 128, 32 of
+// 64), whose other lanes hold zeros.
+enum Rows : int { kRowsElements = 0, kRowsFull = 1, kRowsPadded = 2 };
+
 // Per-lane chunk of one token row: DL values at `p` (K or V plane), converted
-// to fp32. VEC uses 16-byte loads; otherwise element loads masked to `dim`.
-template <int DT, int DL, bool VEC>
+// to fp32. VEC (Rows) uses 16-byte loads; otherwise element loads masked to `dim`.
+// The G lanes of a row take its 16-byte chunks in turn (lane g chunks g, g + G,
+// ..), so that each load instruction covers consecutive bytes also where a lane
+// owns several chunks; with a lane's chunks next to each other fp32 and head
+// dim 128 streamed at 2.1-2.8 TB/s, fp32's 8 x 900 tokens x 25 heads of 128 in
+// 64 us. col_of(i): the column of a lane's value i less its first.
+template <int DT, int DL, int VEC, int G>
 struct Chunk {
+  static __device__ __forceinline__ constexpr int col_of(int i) {
+    return VEC ? i / per16<DT>() * (G * per16<DT>()) + i % per16<DT>() : i;
+  }
+  static __device__ __forceinline__ int first_col(int g) { return VEC ? g * per16<DT>() : g * DL; }
   using T = typename Elem<DT>::T;
   static constexpr int NV = VEC ? DL * elem_bytes<DT>() / 16 : 1;
   u32x4 raw[VEC ? NV : 1];
@@ -288,8 +303,9 @@ struct Chunk {
       const auto* v = global_view(reinterpret_cast<const u32x4*>(p));
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        if constexpr (NTL) raw[i] = __builtin_nontemporal_load(v + i);
-        else raw[i] = v[i];
+        if (VEC == kRowsPadded && col0 + i * G * per16<DT>() >= dim) raw[i] = u32x4{0u, 0u, 0u, 0u};
+        else if constexpr (NTL) raw[i] = __builtin_nontemporal_load(v + i * G);
+        else raw[i] = v[i * G];
       }
     } else {
       const auto* g = global_view(p);
@@ -301,7 +317,7 @@ struct Chunk {
   __device__ __forceinline__ void load_lds(const T* p, int col0, int dim) {
     if constexpr (VEC) {
 #pragma unroll
-      for (int i = 0; i < NV; ++i) raw[i] = reinterpret_cast<const u32x4*>(p)[i];
+      for (int i = 0; i < NV; ++i) raw[i] = reinterpret_cast<const u32x4*>(p)[i * G];
     } else {
 #pragma unroll
       for (int i = 0; i < DL; ++i) val[i] = (col0 + i < dim) ? to_f32<DT>(p[i]) : 0.f;
@@ -334,7 +350,7 @@ struct Chunk {
 // K conversion is needed and the query takes DL/2 registers; the 1/sqrt(D)
 // and log2(e) factors are applied to the summed score. fp32 and the masked
 // path keep a pre-scaled fp32 query.
-template <int DT, int D, bool VEC, int G = kGroup>
+template <int DT, int D, int VEC, int G = kGroup>
 struct Query {
   using T = typename Elem<DT>::T;
   static constexpr int DL = D / G;
@@ -343,7 +359,7 @@ struct Query {
   float qf[PACKED ? 1 : DL];
   float post_scale;
   __device__ __forceinline__ void load(const T* q, int col0, int dim, float scale) {
-    Chunk<DT, DL, VEC> c;
+    Chunk<DT, DL, VEC, G> c;
     c.load(q + col0, col0, dim);
     if constexpr (PACKED) {
 #pragma unroll
@@ -357,7 +373,7 @@ struct Query {
     }
   }
   // This lane's part of q.k (before the group sum and post_scale).
-  __device__ __forceinline__ float partial(const Chunk<DT, DL, VEC>& k) const {
+  __device__ __forceinline__ float partial(const Chunk<DT, DL, VEC, G>& k) const {
     float s = 0.f;
     if constexpr (PACKED) {
       typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -378,7 +394,7 @@ struct Query {
     }
     return s;
   }
-  __device__ __forceinline__ float score(const Chunk<DT, DL, VEC>& k) const {
+  __device__ __forceinline__ float score(const Chunk<DT, DL, VEC, G>& k) const {
     return group_sum<G>(partial(k)) * post_scale;
   }
 };
@@ -388,7 +404,7 @@ struct Query {
 // rb = rb_first, rb_first + rb_step, ... are processed U at a time; with
 // STAGES = 2 the loads of the next U row-blocks are in flight while the
 // current ones are scored and accumulated.
-template <int DT, int D, bool VEC, int U, int STAGES>
+template <int DT, int D, int VEC, int U, int STAGES>
 __device__ __forceinline__ void stream_rows(Softmax<D / kGroup>& st, const Query<DT, D, VEC>& q,
                                             typename Elem<DT>::T const* const* s_page,
                                             int ntok, int rb_first, int rb_step,
@@ -397,10 +413,10 @@ __device__ __forceinline__ void stream_rows(Softmax<D / kGroup>& st, const Query
   constexpr int DL = D / kGroup;
   const int lane = threadIdx.x & (kWave - 1);
   const int tok = lane >> 2;
-  const int col0 = (lane & 3) * DL;
+  const int col0 = Chunk<DT, DL, VEC, kGroup>::first_col(lane & 3);
   const int nrb = (ntok + kRowBlock - 1) / kRowBlock;
   const int pmask = g.page_size - 1;
-  using C = Chunk<DT, DL, VEC>;
+  using C = Chunk<DT, DL, VEC, kGroup>;
   auto issue = [&](int rb0, C* kc, C* vc, bool* valid) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -477,6 +493,9 @@ struct DecodeArgs {
   // other pass reversed. Needs 2 * (batch rounded up to 4) ints of dynamic LDS.
   int rank_rows;
   int rank_per;
+  // > 0: every row attends this many keys (kVisitUniform; offsets is null).
+  // With k null they all lie in the pages, else the last is the new token.
+  int uniform_len;
   // Work list built on the device (order_kernel) for a batch whose rows may
   // split: work_count[0] (row, split) pairs at `work`, then work_count[1]
   // merge rows. `items` is then only the capacity (batch * nsplit_max *
@@ -488,8 +507,9 @@ struct DecodeArgs {
 // instantiation carries only its own prologue (the kernel's start is
 // latency-bound, and measured slower when unused prologue code grew):
 // from a work list (host- or device-built), by ranking the rows in every
-// workgroup, or as the plain (split, row, head) grid.
-constexpr int kVisitList = 0, kVisitRank = 1, kVisitGrid = 2;
+// workgroup, or as the plain (split, row, head) grid, of rows of their own
+// lengths or of one length known to the host.
+constexpr int kVisitList = 0, kVisitRank = 1, kVisitGrid = 2, kVisitUniform = 3;
 
 // Rows a decode workgroup ranks on its own (the ranking costs each thread
 // batch / threads * batch LDS reads).
@@ -505,17 +525,17 @@ constexpr int kOrderThreads = 1024;
 // slot i for page sizes >= 16 (one page per row-block), slots 2i and 2i + 1
 // for page size 8. Page bases are broadcast with readlane (scalar registers)
 // or, for page size 8, a lane shuffle; no LDS and no barrier are involved.
-template <int DT, int D, bool VEC, int U, int STAGES, int G>
+template <int DT, int D, int VEC, int U, int STAGES, int G>
 __device__ __forceinline__ void stream_wave(Softmax<D / G, G>& st, const Query<DT, D, VEC, G>& q,
                                             uint64_t base, int ntok, int wave, int waves,
                                             const Geometry& g, int dim) {
   using T = typename Elem<DT>::T;
   constexpr int DL = D / G;
   constexpr int RB = kWave / G;  // tokens per wave step
-  using C = Chunk<DT, DL, VEC>;
+  using C = Chunk<DT, DL, VEC, G>;
   const int lane = threadIdx.x & (kWave - 1);
   const int tok = lane / G;
-  const int col0 = (lane % G) * DL;
+  const int col0 = Chunk<DT, DL, VEC, G>::first_col(lane % G);
   const int pmask = g.page_size - 1;
   const bool two_pages = g.page_size < RB;
   const int nrb = (ntok + RB - 1) / RB;
@@ -583,9 +603,9 @@ __device__ __forceinline__ void stream_wave(Softmax<D / G, G>& st, const Query<D
 // VGPRs: one VGPR more drops a whole workgroup per compute unit (and the
 // launcher then picks 4-wave workgroups), so the bound is stated. Other
 // shapes need more registers and keep the compiler's choice.
-template <int DT, int D, bool VEC, int U, int STAGES, int WAVES, int G, int MODE>
+template <int DT, int D, int VEC, int U, int STAGES, int WAVES, int G, int MODE>
 __global__ __launch_bounds__(WAVES * kWave)
-__attribute__((amdgpu_waves_per_eu(WAVES == 8 && D == 64 && VEC && DT != kF32 && U <= 2 ? 6 : 1)))
+__attribute__((amdgpu_waves_per_eu(WAVES == 8 && D == 64 && VEC == kRowsFull && DT != kF32 && U <= 2 ? 6 : 1)))
 void decode_kernel(DecodeArgs a) {
   using T = typename Elem<DT>::T;
   constexpr int DL = D / G;
@@ -609,7 +629,7 @@ void decode_kernel(DecodeArgs a) {
   uint64_t tl_entry = 0, tl_loads = 0, tl_barrier = 0, tl_stream = 0;
 #endif
   const Geometry& g = a.g;
-  const int dim = VEC ? D : g.dim;
+  const int dim = VEC == kRowsFull ? D : g.dim;
   const int tid = threadIdx.x;
   const int64_t bh_count = int64_t(a.batch) * g.heads;
   // The slab table of a small pool is staged in LDS. A workgroup whose first
@@ -672,7 +692,7 @@ void decode_kernel(DecodeArgs a) {
   }
   const int wave = tid >> 6;
   const int lane = tid & (kWave - 1);
-  const int col0 = (lane % G) * DL;
+  const int col0 = Chunk<DT, DL, VEC, G>::first_col(lane % G);
   const int64_t cap = int64_t(g.columns) * g.page_size;
   const int sub_shift = g.page_size < RB ? 1 : 0;
   const int rb_per_wave = a.split_tokens / RB / WAVES;
@@ -737,8 +757,9 @@ void decode_kernel(DecodeArgs a) {
     const int64_t qrow = int64_t(b) * a.qkv_stride + int64_t(head) * dim;  // q, k, v row
     qv.load(qp + qrow, col0, dim, a.qscale);
     T new_k{}, new_v{};
-    if (tid < dim) { new_k = kin[qrow + tid]; new_v = vin[qrow + tid]; }
-    const int offset = MODE == kVisitRank ? s_len[b] : a.offsets[b];
+    const bool has_new = MODE != kVisitUniform || a.k;
+    if (has_new && tid < dim) { new_k = kin[qrow + tid]; new_v = vin[qrow + tid]; }
+    const int offset = MODE == kVisitRank ? s_len[b] : MODE == kVisitUniform ? a.uniform_len - 1 : a.offsets[b];
 #ifdef MT_DECODE_TIMELINE
     if (item == blockIdx.x) tl_loads = stamp_after(offset + physical);
 #endif
@@ -755,7 +776,7 @@ void decode_kernel(DecodeArgs a) {
     if (split >= nsplit) continue;
     const int64_t t0 = t0i;
     const int64_t t1 = L < t0 + a.split_tokens ? L : t0 + a.split_tokens;
-    const bool owns_new = L > 0 && split == nsplit - 1;
+    const bool owns_new = has_new && L > 0 && split == nsplit - 1;
     const int ntok_paged = int((owns_new ? t1 - 1 : t1) - t0);  // tokens read from pages
     // Staged in LDS once the loads above are in flight: the slab table (first
     // item only) and the new token's K/V row, which is needed only after the
@@ -766,7 +787,7 @@ void decode_kernel(DecodeArgs a) {
       for (int j = 0; j < SLABS_PER_THREAD; ++j)
         if (tid + j * NT < kLdsSlabs) s_slabs[tid + j * NT] = slab_reg[j];
     }
-    if (tid < dim) { s_new[0][tid] = new_k; s_new[1][tid] = new_v; }
+    if (tid < (VEC == kRowsPadded ? D : dim)) { s_new[0][tid] = new_k; s_new[1][tid] = new_v; }
     __syncthreads();
     slabs_staged = true;
 #ifdef MT_DECODE_TIMELINE
@@ -801,7 +822,7 @@ void decode_kernel(DecodeArgs a) {
       // and written into its page when the page exists (reference append,
       // src/paged_attention_kernel.cu:23-33). A missing page reads as NaN.
       const int64_t pos = L - 1;
-      Chunk<DT, DL, VEC> kn, vn;
+      Chunk<DT, DL, VEC, G> kn, vn;
       kn.load_lds(&s_new[0][col0], col0, dim);
       vn.load_lds(&s_new[1][col0], col0, dim);
       if (lane < G && new_page) {
@@ -809,9 +830,10 @@ void decode_kernel(DecodeArgs a) {
         T* vp = kp + g.kind_stride;
         if constexpr (VEC) {
 #pragma unroll
-          for (int i = 0; i < Chunk<DT, DL, VEC>::NV; ++i) {
-            global_view(reinterpret_cast<u32x4*>(kp))[i] = kn.raw[i];
-            global_view(reinterpret_cast<u32x4*>(vp))[i] = vn.raw[i];
+          for (int i = 0; i < Chunk<DT, DL, VEC, G>::NV; ++i) {
+            if (VEC == kRowsPadded && col0 + i * G * per16<DT>() >= dim) break;
+            global_view(reinterpret_cast<u32x4*>(kp))[i * G] = kn.raw[i];
+            global_view(reinterpret_cast<u32x4*>(vp))[i * G] = vn.raw[i];
           }
         } else {
           for (int i = 0; i < DL && col0 + i < dim; ++i) {
@@ -835,7 +857,7 @@ void decode_kernel(DecodeArgs a) {
     if ((lane & 15) < G) {
       const int si = wave * 4 + row;
 #pragma unroll
-      for (int i = 0; i < DL; ++i) s_acc[si][col0 + i] = st.acc[i];
+      for (int i = 0; i < DL; ++i) s_acc[si][col0 + Chunk<DT, DL, VEC, G>::col_of(i)] = st.acc[i];
       if ((lane & 15) == 0) { s_m[si] = st.m; s_l[si] = st.l; }
     }
     __syncthreads();
@@ -938,7 +960,7 @@ __global__ __launch_bounds__(128) void merge_kernel(DecodeArgs a) {
       }
     };
     load_chunk(0);
-    const int offset = a.offsets[b];
+    const int offset = a.offsets ? a.offsets[b] : a.uniform_len - 1;
     const int64_t L = offset < 0 ? 0 : int64_t(offset) + 1;
     if (L > cap) continue;
     const int nsplit = L == 0 ? 1 : int((L + a.split_tokens - 1) / a.split_tokens);
@@ -1197,17 +1219,17 @@ constexpr int pf_part_row() { return D + 4; }
 // (reference paged_forward with offsets == nullptr, src/paged_attention_kernel.cu:35-85):
 // query qi attends keys kj < nk with kj <= offset + qi. One wave per query,
 // four queries per workgroup; page bases are resolved per 2048-token chunk.
-template <int DT, int D, bool VEC, int U>
+template <int DT, int D, int VEC, int U>
 __global__ __launch_bounds__(kThreads) void query_kernel(QueryArgs a) {
   using T = typename Elem<DT>::T;
   constexpr int DL = D / kGroup;
   __shared__ const T* s_page[kMaxSplitPages];
   const Geometry& g = a.g;
-  const int dim = VEC ? D : g.dim;
+  const int dim = VEC == kRowsFull ? D : g.dim;
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & (kWave - 1);
-  const int col0 = (lane & 3) * DL;
+  const int col0 = Chunk<DT, DL, VEC, kGroup>::first_col(lane & 3);
   const int qblocks = (a.nq + kWaves - 1) / kWaves;
   const T* qp = static_cast<const T*>(a.q);
   T* out = static_cast<T*>(a.out);
@@ -1238,8 +1260,10 @@ __global__ __launch_bounds__(kThreads) void query_kernel(QueryArgs a) {
     st.wave_merge();
     if (has_q && lane < kGroup) {
       T* orow = out + b * a.o_b + head * a.o_h + qi * a.o_r;
-      for (int i = 0; i < DL; ++i)
-        if (col0 + i < dim) orow[col0 + i] = from_f32<DT>(finalize(st.acc[i], st.l));
+      for (int i = 0; i < DL; ++i) {
+        const int c = col0 + Chunk<DT, DL, VEC, kGroup>::col_of(i);
+        if (c < dim) orow[c] = from_f32<DT>(finalize(st.acc[i], st.l));
+      }
     }
     __syncthreads();
   }
@@ -2074,11 +2098,14 @@ size_t workspace_bytes_for(int64_t bh, int nsplit_max) {
   return size_t(bh) * nsplit_max * (128 + 2) * sizeof(float);
 }
 
-// Whether the decode runs its 16-byte-load kernel for these operands.
-bool decode_vec(int d, int dtype, const void* out, const void* q, const void* k, const void* v,
-                int64_t qkv_stride) {
-  return (d == 64 || d == 128) && aligned16(out) && aligned16(q) && aligned16(k) && aligned16(v) &&
-         (qkv_stride * (dtype == kF32 ? 4 : 2)) % 16 == 0;
+// How the decode reads the rows of these operands.
+Rows decode_rows(int d, int dtype, const void* out, const void* q, const void* k, const void* v,
+                 int64_t qkv_stride) {
+  const int esize = dtype == kF32 ? 4 : 2;
+  if ((d * esize) % 16 || !aligned16(out) || !aligned16(q) || !aligned16(k) || !aligned16(v) ||
+      (qkv_stride * esize) % 16)
+    return kRowsElements;
+  return d == 64 || d == 128 ? kRowsFull : kRowsPadded;
 }
 
 // Bytes of split partials a decode launch writes: (max, denominator,
@@ -2113,7 +2140,7 @@ bool two_wave_split_ok(const DecodeArgs& a) {
 
 // Workgroups of decode_kernel<DT, D, VEC, U, kStages, WAVES, G> resident per
 // compute unit (0 if the query fails), looked up once per instantiation.
-template <int DT, int D, bool VEC, int U, int WAVES, int G>
+template <int DT, int D, int VEC, int U, int WAVES, int G>
 int decode_occupancy() {
   static const int per_cu = [] {
     int n = 0;
@@ -2124,24 +2151,28 @@ int decode_occupancy() {
 }
 
 // The instantiation of the launch's visiting mode.
-template <int DT, int D, bool VEC, int U, int WAVES, int G>
+template <int DT, int D, int VEC, int U, int WAVES, int G>
 void launch_decode_mode(const DecodeArgs& a, int64_t blocks, size_t lds) {
   constexpr int NT = WAVES * kWave;
   if (a.work) decode_kernel<DT, D, VEC, U, kStages, WAVES, G, kVisitList><<<grid_for(blocks), NT, lds>>>(a);
+  else if (a.uniform_len) decode_kernel<DT, D, VEC, U, kStages, WAVES, G, kVisitUniform><<<grid_for(blocks), NT, lds>>>(a);
   else if (a.rank_rows) decode_kernel<DT, D, VEC, U, kStages, WAVES, G, kVisitRank><<<grid_for(blocks), NT, lds>>>(a);
   else decode_kernel<DT, D, VEC, U, kStages, WAVES, G, kVisitGrid><<<grid_for(blocks), NT, lds>>>(a);
 }
 
-template <int DT, int D, bool VEC, int WAVES, int G>
+template <int DT, int D, int VEC, int WAVES, int G>
 hipError_t launch_decode_w(const DecodeArgs& a, int64_t blocks, int unroll) {
   // Row bytes per lane bound the useful unroll: register stages beyond it spill.
-  constexpr int kMaxUnroll = !VEC ? 1 : (D * elem_bytes<DT>() >= 256 ? 2 : 4);
+  constexpr int kMaxUnroll = !VEC ? 1 : (VEC == kRowsPadded || D * elem_bytes<DT>() >= 256 ? 2 : 4);
   constexpr int NT = WAVES * kWave;
   if (unroll == 0) {
     if constexpr (G == 8) {
       // Two row-blocks per register stage: measured best or within 1 % of
-      // the best at every decode shape of configs 2, 4 and 5.
-      unroll = 2;
+      // the best at every decode shape of configs 2, 4 and 5. A grid of at
+      // most one 8-wave workgroup per compute unit has registers for four,
+      // which keep twice the bytes in flight: one row of 1000 tokens x 16
+      // heads bf16 8.8 against 9.5 us, 4 rows to 500 x 25 heads 7.5 against 8.0.
+      unroll = WAVES == 8 && kMaxUnroll >= 4 && blocks <= device_compute_units() ? 4 : 2;
     } else if constexpr (kMaxUnroll >= 4) {
       // The deepest unroll when the whole grid is resident at its
       // occupancy (more loads in flight per wave), else unroll 1, whose
@@ -2191,7 +2222,7 @@ hipError_t launch_decode_w(const DecodeArgs& a, int64_t blocks, int unroll) {
 // more than two residency rounds (finer-grained hand-out of the tail; config
 // 5: 261-263 us vs 267 us with 4; config 4's layer, 2048 workgroups that 2
 // waves would make resident at once, took 9 % longer per step with 2).
-template <int DT, int D, bool VEC>
+template <int DT, int D, int VEC>
 hipError_t launch_decode_t(const DecodeArgs& a, int64_t blocks, int unroll, int waves) {
   constexpr int G = kDecodeGroup;
   constexpr int U8 = VEC && G == 8 ? 2 : 1;
@@ -2208,10 +2239,28 @@ hipError_t launch_decode_t(const DecodeArgs& a, int64_t blocks, int unroll, int 
 }
 
 template <int DT>
-hipError_t launch_decode_dt(const DecodeArgs& a, int64_t blocks, bool vec, int d, int unroll, int waves) {
-  if (vec && d == 64) return launch_decode_t<DT, 64, true>(a, blocks, unroll, waves);
-  if (vec && d == 128) return launch_decode_t<DT, 128, true>(a, blocks, unroll, waves);
-  return launch_decode_t<DT, 128, false>(a, blocks, 1, waves);
+hipError_t launch_decode_dt(const DecodeArgs& a, int64_t blocks, Rows rows, int d, int unroll, int waves) {
+  if (rows == kRowsFull && d == 64) return launch_decode_t<DT, 64, kRowsFull>(a, blocks, unroll, waves);
+  if (rows == kRowsFull) return launch_decode_t<DT, 128, kRowsFull>(a, blocks, unroll, waves);
+  if (rows == kRowsPadded && d < 64) return launch_decode_t<DT, 64, kRowsPadded>(a, blocks, unroll, waves);
+  if (rows == kRowsPadded) return launch_decode_t<DT, 128, kRowsPadded>(a, blocks, unroll, waves);
+  return launch_decode_t<DT, 128, kRowsElements>(a, blocks, 1, waves);
+}
+
+// Split length of a decode of bh (row, head) pairs whose longest context is
+// `longest` tokens, where the library chooses: choose_split's, unless that
+// leaves compute units idle. Then enough splits for two workgroups per
+// compute unit, but no split below kSplitBytes of K and V (a split's own
+// prologue and its share of the merge take about 5 us, in which a workgroup
+// streams that much). One row of 8000 tokens x 12 heads fp16: 12.0 us at 512
+// tokens a split, 13.4 at 1024, 15.2 at 128; 8 rows to 1500: 12.6 against 13.4.
+constexpr int64_t kSplitBytes = 128 * 1024;
+int idle_split(int64_t bh, int64_t longest, int d, int dtype) {
+  const int S = choose_split(longest, 0);
+  const int64_t row_bytes = int64_t(2) * d * (dtype == kF32 ? 4 : 2);
+  const int64_t least = (kSplitBytes / row_bytes + 63) / 64 * 64;
+  const int64_t want = (longest * bh / (2 * std::max(1, device_compute_units())) + 63) / 64 * 64;
+  return int(std::min<int64_t>(S, std::max(least, want)));
 }
 
 int decode_common(void* out, const void* q, const void* k, const void* v, const uint64_t* slabs,
@@ -2234,8 +2283,8 @@ int decode_common(void* out, const void* q, const void* k, const void* v, const 
     return hipErrorInvalidValue;
   if (work && work_items == 0) return hipSuccess;
   const int64_t stride = qkv_stride ? qkv_stride : int64_t(h) * d;
-  const bool vec = decode_vec(d, dtype, out, q, k, v, stride);
-  if (nsplit_max > 1 && (!workspace || workspace_bytes < partial_bytes(bh, nsplit_max, vec, d)))
+  const Rows rows = decode_rows(d, dtype, out, q, k, v, stride);
+  if (nsplit_max > 1 && (!workspace || workspace_bytes < partial_bytes(bh, nsplit_max, rows == kRowsFull, d)))
     return hipErrorInvalidValue;
   DecodeArgs a{};
   a.out = out; a.q = q; a.k = k; a.v = v; a.slabs = slabs; a.table = table; a.offsets = offsets;
@@ -2252,7 +2301,9 @@ int decode_common(void* out, const void* q, const void* k, const void* v, const 
   a.merge_rows = work ? merge_rows : 0;
   // Entries without a work list visit rows longest first when every row has
   // one split and the batch is small enough to rank in each workgroup.
-  if (rank_order && !work && nsplit_max == 1 && b <= kRankRows) {
+  // Where every workgroup has a compute unit to itself the order does not
+  // matter, and the ranking only lengthens the prologue.
+  if (rank_order && !work && nsplit_max == 1 && b <= kRankRows && bh > device_compute_units()) {
     a.rank_rows = 1;
     a.rank_per = std::max(1, device_compute_units() / h);
   } else if (rank_order && !work && order) {
@@ -2273,9 +2324,9 @@ int decode_common(void* out, const void* q, const void* k, const void* v, const 
       a.items = bh;
     }
   }
-  if (dtype == kF32) return launch_decode_dt<kF32>(a, a.items, vec, d, unroll, waves);
-  if (dtype == kF16) return launch_decode_dt<kF16>(a, a.items, vec, d, unroll, waves);
-  if (dtype == kBF16) return launch_decode_dt<kBF16>(a, a.items, vec, d, unroll, waves);
+  if (dtype == kF32) return launch_decode_dt<kF32>(a, a.items, rows, d, unroll, waves);
+  if (dtype == kF16) return launch_decode_dt<kF16>(a, a.items, rows, d, unroll, waves);
+  if (dtype == kBF16) return launch_decode_dt<kBF16>(a, a.items, rows, d, unroll, waves);
   return hipErrorInvalidValue;
 }
 
@@ -2283,8 +2334,14 @@ int decode_common(void* out, const void* q, const void* k, const void* v, const 
 // order (batches past the in-workgroup ranking, or rows that may split, up to
 // kOrderRows rows), and the bytes it writes: the count pair, the (row, split)
 // list and the merge rows.
-bool device_order(int b, int64_t nsplit_max) {
-  return b <= kOrderRows && (nsplit_max > 1 || b > kRankRows) && int64_t(b) * nsplit_max <= INT32_MAX / 2;
+// Not for grids of few rounds of the compute units: the launch (8 us) costs
+// more than the order saves (40 rows to 3000 tokens x 25 heads fp16, 3000
+// workgroups: 71.4 us in batch order, 77.2 with it; 512 rows to 8192 x 25
+// heads, 102,400: 334 against 270).
+constexpr int kOrderBlocksPerUnit = 16;
+bool device_order(int b, int h, int64_t nsplit_max) {
+  return b <= kOrderRows && (nsplit_max > 1 || b > kRankRows) && int64_t(b) * nsplit_max <= INT32_MAX / 2 &&
+         int64_t(b) * h * nsplit_max > int64_t(kOrderBlocksPerUnit) * device_compute_units();
 }
 size_t order_bytes(int b, int64_t nsplit_max) {
   return size_t(2 + 2 * int64_t(b) * nsplit_max + b) * sizeof(int);
@@ -2318,7 +2375,9 @@ struct ThreadWorkspaces {
 };
 thread_local ThreadWorkspaces t_workspaces;
 
-int library_workspace(size_t bytes, void** out) {
+// `capturing` false: not grown while the stream is captured (the allocation
+// would belong to the graph).
+int library_workspace(size_t bytes, void** out, bool capturing = true) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
@@ -2326,6 +2385,11 @@ int library_workspace(size_t bytes, void** out) {
   if (ws.size() <= size_t(dev)) ws.resize(dev + 1, {nullptr, 0});
   auto& slot = ws[dev];
   if (slot.second < bytes) {
+    if (!capturing) {
+      hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(hipStreamPerThread, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
+        return hipErrorOutOfMemory;
+    }
     void* p = nullptr;
     e = hipMallocAsync(&p, bytes, hipStreamPerThread);
     if (e != hipSuccess) {
@@ -2374,6 +2438,43 @@ int scratch_address(void** out) {
   }
   *out = addresses[dev];
   return hipSuccess;
+}
+
+// One query per request over `len` keys, on the decode kernel: every key from
+// the pages (k null), or the last one appended from the k/v rows. out is [b,
+// h * d]. hipErrorNotSupported where the rows need element loads or there is
+// no room for the partials.
+hipError_t decode_uniform(void* out, const void* q, const void* k, const void* v, const uint64_t* slabs,
+                          const int* table, int b, int len, int64_t qkv_stride, int dtype, const Geometry& g) {
+  const Rows rows = decode_rows(g.dim, dtype, out, q, k, v, qkv_stride);
+  if (rows == kRowsElements) return hipErrorNotSupported;
+  const int64_t bh = int64_t(b) * g.heads;
+  const int row_bytes = 2 * g.dim * (dtype == kF32 ? 4 : 2);
+  // Unsplit while a row is short or the rows fill the compute units: the
+  // merge is a launch of its own (1000 tokens x 16 heads bf16, 256 KB a row:
+  // 8.8 us unsplit, 10.1 split; 700 x 12 fp32, 358 KB: 14.7 against 10.4).
+  const bool whole = len <= kMaxSplitTokens &&
+                     (int64_t(len) * row_bytes <= 300 * 1024 || bh >= device_compute_units());
+  DecodeArgs a{};
+  const int most = whole ? len : idle_split(bh, len, g.dim, dtype);
+  const int pieces = (len + most - 1) / most;  // of even length
+  a.split_tokens = ((len + pieces - 1) / pieces + 63) / 64 * 64;
+  a.nsplit_max = (len + a.split_tokens - 1) / a.split_tokens;
+  if (a.nsplit_max > 1) {
+    void* ws = nullptr;
+    if (library_workspace(workspace_bytes_for(bh, a.nsplit_max), &ws, false) != hipSuccess) return hipErrorNotSupported;
+    a.partials = static_cast<float*>(ws);
+  }
+  a.out = out; a.q = q; a.k = k; a.v = v; a.slabs = slabs; a.table = table;
+  a.batch = b; a.uniform_len = len;
+  a.qscale = (1.0f / std::sqrt(float(g.dim))) * kLog2e;
+  a.items = bh * a.nsplit_max;
+  if (a.items > INT32_MAX) return hipErrorNotSupported;
+  a.g = g;
+  a.qkv_stride = qkv_stride;
+  if (dtype == kF32) return launch_decode_dt<kF32>(a, a.items, rows, g.dim, 0, 0);
+  if (dtype == kF16) return launch_decode_dt<kF16>(a, a.items, rows, g.dim, 0, 0);
+  return launch_decode_dt<kBF16>(a, a.items, rows, g.dim, 0, 0);
 }
 
 // Launch of the append kernel for any source strides; the 16-byte path needs
@@ -2536,7 +2637,7 @@ hipError_t launch_query(QueryArgs& a, int dtype) {
       void* ws = nullptr;
       // Without room for the partials the launch runs unsplit.
       if (pieces > 1 && library_workspace(size_t(bh) * items.tiles * pieces * tq * (d <= 64 ? 68 : 132) * sizeof(float),
-                                          &ws) == hipSuccess) {
+                                          &ws, false) == hipSuccess) {
         items.pieces = pieces;
         items.share = plan.share;
         a.partials = static_cast<float*>(ws);
@@ -2606,6 +2707,10 @@ int mt_paged_attention(void* out, const void* q, const uint64_t* slabs, const in
   a.q_b = a.o_b = int64_t(h) * nq * d;
   a.q_h = a.o_h = int64_t(nq) * d;
   a.q_r = a.o_r = d;
+  if (nq == 1) {
+    const hipError_t e = decode_uniform(out, q, nullptr, nullptr, slabs, table, b, nk, int64_t(h) * d, dtype, a.g);
+    if (e != hipErrorNotSupported) return e;
+  }
   return launch_query(a, dtype);
 }
 
@@ -2629,6 +2734,11 @@ int mt_paged_prefill(void* out, const void* q, const void* k, const void* v, con
   a.g = make_geometry(h, d, page_size, pages_per_slab, num_slabs, columns, layer);
   a.q_b = int64_t(n) * qkv_stride; a.q_h = d; a.q_r = qkv_stride;
   a.o_b = int64_t(n) * out_stride; a.o_h = d; a.o_r = out_stride;
+  if (n == 1 && out_stride == hd) {
+    // one token: append and attention in the decode's one launch
+    const hipError_t e = decode_uniform(out, q, k, v, slabs, table, b, offset + 1, qkv_stride, dtype, a.g);
+    if (e != hipErrorNotSupported) return e;
+  }
   if (causal_kernel_takes(a, dtype) && aligned16(k) && aligned16(v)) {
     // The prefill kernel reads the new keys from k/v and writes them to
     // their pages itself: no separate append.
@@ -2760,7 +2870,7 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
       // Without room for the partials the launch runs unsplit.
       pairs = cut(true);
       if (most > 65535 ||
-          (slots && library_workspace(size_t(slots) * h * tq * (d <= 64 ? 68 : 132) * sizeof(float), &ws) != hipSuccess)) {
+          (slots && library_workspace(size_t(slots) * h * tq * (d <= 64 ? 68 : 132) * sizeof(float), &ws, false) != hipSuccess)) {
         share = slots = 0;
         mg = RaggedMerge{};
       }
@@ -2822,9 +2932,9 @@ int mt_paged_decode_batch(void* out, const void* q, const void* k, const void* v
     return hipErrorInvalidValue;
   if (dtype < 0 || dtype > 2) return hipErrorInvalidValue;
   const int64_t cap = int64_t(columns) * page_size;
-  const int S = choose_split(cap, 0);
+  const int S = cap > kDefaultSplitTokens ? idle_split(int64_t(b) * h, cap, d, dtype) : choose_split(cap, 0);
   const int64_t nsplit_max = (cap + S - 1) / S;
-  const bool ordered = device_order(b, nsplit_max);
+  const bool ordered = device_order(b, h, nsplit_max);
   // Workspace: split partials, then the device-built visiting order.
   const size_t part = nsplit_max > 1 ? align256(workspace_bytes_for(int64_t(b) * h, int(nsplit_max))) : 0;
   const size_t ws_bytes = part + (ordered ? order_bytes(b, nsplit_max) : 0);
@@ -2849,12 +2959,12 @@ int mt_paged_decode_batch_noalloc(void* out, const void* q, const void* k, const
     return hipErrorInvalidValue;
   if (dtype < 0 || dtype > 2) return hipErrorInvalidValue;
   const int64_t cap = int64_t(columns) * page_size;
-  const int S = choose_split(cap, 0);
+  const int S = cap > kDefaultSplitTokens ? idle_split(int64_t(b) * h, cap, d, dtype) : choose_split(cap, 0);
   const int64_t nsplit_max = (cap + S - 1) / S;
-  const bool ordered = device_order(b, nsplit_max);
+  const bool ordered = device_order(b, h, nsplit_max);
   // The fixed array holds the split partials, then the device-built visiting
   // order; a shape that needs more is refused before any launch.
-  const bool vec = decode_vec(d, dtype, out, q, k, v, int64_t(h) * d);
+  const bool vec = decode_rows(d, dtype, out, q, k, v, int64_t(h) * d) == kRowsFull;
   const size_t part = nsplit_max > 1 ? align256(partial_bytes(int64_t(b) * h, nsplit_max, vec, d)) : 0;
   const size_t need = part + (ordered ? order_bytes(b, nsplit_max) : 0);
   if (need > kNoAllocScratchBytes) return hipErrorInvalidValue;
