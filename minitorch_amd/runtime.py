@@ -128,10 +128,15 @@ def runtime():
 
 def call(lib, name, signature, *args):
     """Call an ``int mt_*`` entry point and raise on a nonzero status
-    (reference minitorch/cuda_resident_ops.py:41-44)."""
+    (reference minitorch/cuda_resident_ops.py:41-44). The signature is set only
+    where the entry point holds another one: ctypes builds converters for every
+    argument when it is set, about half of a call's host time."""
     f = getattr(lib, name)
-    f.argtypes, f.restype = signature, I
-    runtime().check(f(*args))
+    if f.argtypes != signature or f.restype is not I:
+        f.argtypes, f.restype = signature, I
+    status = f(*args)
+    if status:
+        runtime().check(status)
 
 
 class RawDeviceBuffer:
