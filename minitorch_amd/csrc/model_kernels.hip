@@ -647,6 +647,11 @@ __global__ __launch_bounds__(1024) void projection_kernel(ProjArgs p) {
   constexpr int SMAX = proj_max_steps<MT * NT>();
   constexpr int NL = NT + MT;  // 16-byte loads per lane and step
   constexpr int NQ = NT * MT;  // output tiles
+  // outputs a finishing thread takes: few tiles are spread over up to four
+  // times the threads that hold them, eight keep theirs (of two features a
+  // thread, 12 waves would have a second turn: 100 rows x 768 4 % slower)
+  constexpr int R = NQ >= 8 ? 4 : NQ >= 4 ? 2 : 1;
+  struct alignas(R * sizeof(T)) Outputs { T v[R]; };
   constexpr bool LN = PS >= 0;
   constexpr bool XT = (LAY & kProjXTiled) != 0;
   constexpr int XSTEP = XT ? 512 : 32;  // elements between a lane's activations of consecutive 32-wide steps
@@ -686,11 +691,14 @@ __global__ __launch_bounds__(1024) void projection_kernel(ProjArgs p) {
       xoff[t] = row * p.k + k0;
     }
   }
-  // the bias of the output tile this wave finishes first (q = wave), loaded
-  // with the operands instead of after the reduction
-  uint2 bias0 = uint2{0u, 0u};
-  if (EPI != kProjPartials && p.bias && wave < NQ)
-    bias0 = *reinterpret_cast<const uint2*>(static_cast<const T*>(p.bias) + f0 + 16 * (wave / MT) + 4 * grp);
+  // the bias of the outputs this thread finishes first, loaded with the
+  // operands instead of after the reduction
+  Outputs bias0{};
+  if (EPI != kProjPartials && p.bias && int(threadIdx.x) < NQ * 256 / R) {
+    const int e = int(threadIdx.x);
+    bias0 = *reinterpret_cast<const Outputs*>(static_cast<const T*>(p.bias) + f0 + 16 * (e / (256 / R) / MT) +
+                                              R * (e & (16 / R - 1)));
+  }
   u32x4 buf[SMAX][NL];
   if constexpr (LN) {
     float* vbuf = reinterpret_cast<float*>(red + waves * 64);
@@ -733,36 +741,54 @@ __global__ __launch_bounds__(1024) void projection_kernel(ProjArgs p) {
     }
   }
 
+  // The waves' sums meet in LDS, where 4-feature group g of tile column c lies
+  // in chunk 16 g + (c ^ 4 g): the finishing threads take R consecutive
+  // features each, 16 features of a row side by side, and read without bank
+  // conflicts. The tail after the barrier is a chain of LDS reads, adds and
+  // the epilogue, with nothing else of the workgroup to cover it: finished by
+  // one wave per tile, 4 features a lane, the other waves idle and the chain
+  // is four times as long. us per launch, that against this: 4 split sums of
+  // [8, 768] fp16 3.60 and 3.26, QKV of 8 rows 6.09 and 5.58, fc with GELU of
+  // 40 rows x 1024 bf16 6.06 and 5.86, its down projection 5.48 and 5.36.
+  // Both projections of the MLP, per call: 40 rows x 1024 12.26 and 11.81, 128
+  // rows 16.64 and 15.98, 8 rows x 768 9.16 and 8.12.
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) red[(wave * NQ + q) * 64 + lane] = acc[q];
+  for (int q = 0; q < NQ; ++q) red[(wave * NQ + q) * 64 + (lane ^ (4 * grp))] = acc[q];
   __syncthreads();
-  for (int q = wave; q < NQ; q += waves) {
-    floatx4 a = red[q * 64 + lane];
-    for (int v = 1; v < waves; ++v) {
-      const floatx4 b = red[(v * NQ + q) * 64 + lane];
-      a[0] += b[0]; a[1] += b[1]; a[2] += b[2]; a[3] += b[3];
-    }
-    const int row = r0 + 16 * (q % MT) + col;
+  const float* sums = reinterpret_cast<const float*>(red);
+  for (int e = int(threadIdx.x); e < NQ * 256 / R; e += int(blockDim.x)) {
+    const int q = e / (256 / R), c = e / (16 / R) & 15, f = R * (e & (16 / R - 1));
+    const int row = r0 + 16 * (q % MT) + c;
     if (row >= p.m) continue;
-    const int feat = f0 + 16 * (q / MT) + 4 * grp;
-    float v[4] = {a[0], a[1], a[2], a[3]};
+    const int at = q * 256 + 64 * (f >> 2) + 4 * (c ^ (f & 12)) + (f & 3);
+    float v[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) v[i] = sums[at + i];
+#pragma unroll 5
+    for (int o = 1; o < waves; ++o)
+#pragma unroll
+      for (int i = 0; i < R; ++i) v[i] += sums[o * NQ * 256 + at + i];
+    const int feat = f0 + 16 * (q / MT) + f;
     if constexpr (EPI == kProjPartials) {
-      float* o = static_cast<float*>(p.out) + (int64_t(blockIdx.y) * p.m + row) * p.n + feat;
-      *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[2], v[3]};
+      struct alignas(R * sizeof(float)) Sums { float v[R]; } y;
+#pragma unroll
+      for (int i = 0; i < R; ++i) y.v[i] = v[i];
+      *reinterpret_cast<Sums*>(static_cast<float*>(p.out) + (int64_t(blockIdx.y) * p.m + row) * p.n + feat) = y;
     } else {
       if (p.bias) {
-        const uint2 b = q == wave ? bias0 : *reinterpret_cast<const uint2*>(static_cast<const T*>(p.bias) + feat);
-        v[0] += to_f32<DT>(T(b.x & 0xffffu)); v[1] += to_f32<DT>(T(b.x >> 16));
-        v[2] += to_f32<DT>(T(b.y & 0xffffu)); v[3] += to_f32<DT>(T(b.y >> 16));
+        if (e != int(threadIdx.x)) bias0 = *reinterpret_cast<const Outputs*>(static_cast<const T*>(p.bias) + feat);
+#pragma unroll
+        for (int i = 0; i < R; ++i) v[i] += to_f32<DT>(bias0.v[i]);
       }
       if constexpr (EPI == kProjGelu) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = gelu_tanh(v[i]);
+        for (int i = 0; i < R; ++i) v[i] = gelu_tanh(v[i]);
       }
       T* o = static_cast<T*>(p.out) + ((LAY & kProjOutTiled) ? tiled_offset(row, feat, p.n) : int64_t(row) * p.n + feat);
-      *reinterpret_cast<uint2*>(o) =
-          uint2{uint32_t(from_f32<DT>(v[0])) | (uint32_t(from_f32<DT>(v[1])) << 16),
-                uint32_t(from_f32<DT>(v[2])) | (uint32_t(from_f32<DT>(v[3])) << 16)};
+      Outputs y;
+#pragma unroll
+      for (int i = 0; i < R; ++i) y.v[i] = from_f32<DT>(v[i]);
+      *reinterpret_cast<Outputs*>(o) = y;
     }
   }
 }

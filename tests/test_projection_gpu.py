@@ -102,6 +102,16 @@ def test_decode_projection(dtype, m, n, k, splits, epilogue):
     assert np.all(np.abs(got - ref) <= tol), float(np.max(np.abs(got - ref) / tol))
 
 
+# one to nine waves to sum, every tile shape (1, 2, 4 and 8 output tiles, by
+# rows and by n % 32), with fewer threads than outputs and with more
+@pytest.mark.parametrize('epilogue', [0, 1, 2])
+@pytest.mark.parametrize('k', [32, 96, 288])
+@pytest.mark.parametrize('m,n', [(1, 16), (15, 48), (17, 32), (32, 48), (33, 64), (63, 48), (65, 48), (65, 64),
+                                 (128, 32), (129, 48)])
+def test_sums_of_few_waves(m, n, k, epilogue):
+    test_decode_projection('bfloat16', m, n, k, 1, epilogue)
+
+
 @pytest.mark.parametrize('dtype', ['bfloat16', 'float16'])
 def test_decode_projection_without_bias(dtype):
     rng = np.random.default_rng(7)
