@@ -654,6 +654,16 @@ __global__ __launch_bounds__(1024) void projection_kernel(ProjArgs p) {
   struct alignas(R * sizeof(T)) Outputs { T v[R]; };
   constexpr bool LN = PS >= 0;
   constexpr bool XT = (LAY & kProjXTiled) != 0;
+  // Row-major activations of several row tiles: consecutive lanes load along a
+  // row (lane l: row l / 4, 16 bytes l % 4), which the memory pipeline
+  // coalesces, and trade places in LDS. Loaded in operand order (lane l: row
+  // l % 16) a fragment is 64 separate 16-byte pieces to it, a third of the rate
+  // a compute unit takes in otherwise. Both projections of an MLP, us per call
+  // in operand order and traded (bf16): 40 rows x 1024 11.81 and 11.02, 128
+  // rows 15.98 and 14.38, 128 rows x 768 12.95 and 10.97, 32 rows 9.00 and
+  // 8.35; at one row tile, whose loads are few, the trade's LDS round trip
+  // would stand alone in the chain, so it keeps operand order.
+  constexpr bool TRADE = !XT && !LN && MT >= 2;
   constexpr int XSTEP = XT ? 512 : 32;  // elements between a lane's activations of consecutive 32-wide steps
   static_assert(!LN || (MT == 1 && NT == 1), "the LayerNorm prologue takes one row and one feature tile");
   static_assert(!LN || LAY == 0, "the LayerNorm prologue reads its activations from LDS");
@@ -687,8 +697,8 @@ __global__ __launch_bounds__(1024) void projection_kernel(ProjArgs p) {
     // rows past m repeat row m - 1
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      const int row = r0 + 16 * t + col < p.m ? r0 + 16 * t + col : p.m - 1;
-      xoff[t] = row * p.k + k0;
+      const int at = r0 + 16 * t + (TRADE ? lane >> 2 : col);
+      xoff[t] = (at < p.m ? at : p.m - 1) * p.k + (TRADE ? k0 - 8 * grp + 8 * (lane & 3) : k0);
     }
   }
   // the bias of the outputs this thread finishes first, loaded with the
@@ -732,6 +742,20 @@ __global__ __launch_bounds__(1024) void projection_kernel(ProjArgs p) {
 #pragma unroll
   for (int s = 0; s < SMAX; ++s) {
     if (s < steps) {
+      if constexpr (TRADE) {
+        // through the wave's own part of the LDS, whose accesses a wave's are
+        // in order; row r's chunk c lies at 4 r + (c ^ r / 4), so that neither
+        // side has bank conflicts
+        u32x4* own = reinterpret_cast<u32x4*>(red) + wave * NQ * 64;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) own[64 * t + (lane ^ (lane >> 4))] = buf[s][NT + t];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) buf[s][NT + t] = own[64 * t + 4 * col + (grp ^ (col >> 2))];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
 #pragma unroll
       for (int f = 0; f < NT; ++f)
 #pragma unroll
