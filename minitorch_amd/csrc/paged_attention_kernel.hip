@@ -33,8 +33,8 @@
 //
 // Causal attention of several queries per request (a prefill) runs on the
 // matrix cores for every type and head dims of whole 16-byte chunks
-// (causal_kernel: 32 queries a wave, S^T = K Q^T and O^T += V^T P^T); a single
-// query and the shapes it does not take use the per-query query_kernel.
+// (causal_kernel: 32 queries a wave, S^T = K Q^T and O^T += V^T P^T), a single
+// query on the decode kernel; other rows use the per-query query_kernel.
 #include "mt_device.h"
 #include "../../include/mt_paged.h"
 #include <algorithm>
@@ -1325,7 +1325,7 @@ struct AppendArgs {
 constexpr int kPfWindowPages = 512;  // page bases resolved into LDS at a time
 constexpr int kPfBlock = 64;         // keys per unit of a split over workgroups
 constexpr float kRescale = 6.f;
-constexpr int kPfMinQueries = 2;     // fewer queries use query_kernel
+constexpr int kPfMinQueries = 2;     // a single query runs the decode kernel or query_kernel
 
 // x of lanes l and l ^ 32 (in either order): the permlane swap of two copies
 // of x leaves x[l % 32] in one and x[l % 32 + 32] in the other.
@@ -2613,8 +2613,8 @@ void launch_causal(int config, int dtype, int64_t items_count, const QueryArgs& 
   else launch_causal_dt<kBF16>(config, blocks, a, items);
 }
 
-// Causal attention launch for any q/out strides: the matrix-core prefill
-// kernel where prefill_kernel_takes, the per-query kernel otherwise (which
+// Causal attention launch for any q/out strides: the matrix-core causal
+// kernel where causal_kernel_takes, the per-query kernel otherwise (which
 // reads every key from the pages: a.k must then be null).
 hipError_t launch_query(QueryArgs& a, int dtype) {
   const int d = a.g.dim;

@@ -1,9 +1,9 @@
 """GPU parity of causal paged prefill attention (``mt_paged_attention``)
 against the float64 oracle.
 
-For fp16/bf16 with head_dim 64 or 128 and at least 16 queries the library
-runs the matrix-core prefill kernel; the other shapes run the per-query
-kernel. Both follow reference paged_forward with offsets == nullptr
+Rows of whole, aligned 16-byte chunks run the matrix-core causal kernel (two
+or more queries) or the decode kernel (one); the others run the per-query
+kernel. All follow reference paged_forward with offsets == nullptr
 (src/paged_attention_kernel.cu:35-85): nk = offset + nq, query qi attends
 keys kj <= offset + qi, and a missing page gives NaN for every query that
 attends it. Page sizes are 8, 16 and 32 (the entry point rejects others). Tolerances are in tests/tolerances.py.
@@ -137,8 +137,8 @@ def test_prefill_large_scores(dtype):
 
 
 def test_prefill_matches_per_query_kernel_below_threshold():
-    # 15 queries run the per-query kernel, 16 the matrix-core kernel; both
-    # against the oracle on the same pages.
+    # 15 and 16 queries (once the two sides of the matrix-core kernel's
+    # threshold) against the oracle on the same pages.
     case = prefill_case(47, batch=2, heads=2, dim=64, page_size=16, nk=60, dtype='float16')
     dev = DevicePagedCase(case)
     run_prefill(case, 15, 59, 44, seed=9, dev=dev)
