@@ -2375,8 +2375,9 @@ struct ThreadWorkspaces {
 };
 thread_local ThreadWorkspaces t_workspaces;
 
-// `capturing` false: not grown while the stream is captured (the allocation
-// would belong to the graph).
+// `capturing` false: refused while the stream is captured. A buffer grown
+// there would belong to the graph, and a later call that grows the buffer
+// frees the one that the graph's replays would still write to.
 int library_workspace(size_t bytes, void** out, bool capturing = true) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -2384,12 +2385,12 @@ int library_workspace(size_t bytes, void** out, bool capturing = true) {
   auto& ws = t_workspaces.per_device;
   if (ws.size() <= size_t(dev)) ws.resize(dev + 1, {nullptr, 0});
   auto& slot = ws[dev];
+  if (!capturing) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(hipStreamPerThread, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
+      return hipErrorOutOfMemory;
+  }
   if (slot.second < bytes) {
-    if (!capturing) {
-      hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-      if (hipStreamIsCapturing(hipStreamPerThread, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
-        return hipErrorOutOfMemory;
-    }
     void* p = nullptr;
     e = hipMallocAsync(&p, bytes, hipStreamPerThread);
     if (e != hipSuccess) {
