@@ -1512,7 +1512,7 @@ __device__ __forceinline__ float inverse(float l) { return l > 0.f ? 1.f / l : (
 template <int DT>
 __device__ __forceinline__ float divided(float acc, float l, float inv) {
   const float x = acc * inv;
-  if constexpr (DT == kF32) return fmaf(fmaf(-x, l, acc), inv, x);
+  if constexpr (DT == kF32) return fabsf(x) < INFINITY ? fmaf(fmaf(-x, l, acc), inv, x) : x;
   else return x;
 }
 
@@ -1540,6 +1540,108 @@ __device__ __forceinline__ const char* uniform(const char* p) {
 template <int N>
 __device__ __forceinline__ void wait_staged() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
+// Queries of item `item` (tiles of TQ) that the matrix cores left non-finite,
+// a bit each of 32-query group t in `left`: every WAVES-th of them from the
+// `wave`-th on is attended once more, by one wave on the VALU, over the keys it
+// attends and no others. On the matrix cores a key that a query does not attend
+// has weight 0, and 0 * Inf or 0 * NaN of its V is NaN; so is the 0 * Inf of a
+// weight's low part. For kernels whose arguments are (QueryArgs, Items): they
+// are read anew, and the walk is kept small (a lane scores a key, then holds one
+// or two columns of the output), so that this rare path costs the kernel's own
+// no registers. Finite calls, us without and with the check: 16 prompts of
+// 32-512 tokens fp16 19.6 and 19.6, 4 x 333 tokens fp32 25.6 and 26.1.
+template <int DT, int DP, int TQ, int WAVES, class Items, bool FUSED>
+__device__ __forceinline__ void attend_again(int64_t item, int t, int wave, uint32_t left) {
+  using T = typename Elem<DT>::T;
+  constexpr int E = per16<DT>(), COLS = DP / kWave;
+  struct Args { QueryArgs a; Items items; };
+  uint64_t at = reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(at));
+  const QueryArgs& a = reinterpret_cast<const Args*>(at)->a;
+  const Geometry& g = a.g;
+  PfItem it;
+  reinterpret_cast<const Args*>(at)->items.get(item, a, TQ, it);
+  int lane = threadIdx.x & (kWave - 1);
+  asm volatile("" : "+v"(lane));
+  const int kend = it.offset + ((it.tile + 1) * TQ < it.nq ? (it.tile + 1) * TQ : it.nq);
+  const int kstop = int64_t(it.kb1) * kPfBlock < kend ? it.kb1 * kPfBlock : kend;
+#pragma unroll 1
+  for (int turn = 0; left; left &= left - 1, ++turn) {
+    if (turn % WAVES != wave) continue;
+    const int q = 32 * t + __builtin_ctz(left);
+    const int row = it.tile * TQ + q;
+    const int k1 = min(kstop, it.offset + row + 1);
+    const T* qrow = static_cast<const T*>(a.q) + it.q0 + row * a.q_r;
+    float m = -INFINITY, l = 0.f, acc[COLS];
+#pragma unroll
+    for (int e = 0; e < COLS; ++e) acc[e] = 0.f;
+#pragma unroll 1
+    for (int k0 = it.kb0 * kPfBlock; k0 < k1; k0 += kWave) {
+      const int key = k0 + lane;
+      const T* page = key < k1 ? page_base<T>(a.slabs, it.table_row, key >> g.log2_page, g, it.head) : nullptr;
+      const T *kp = nullptr, *vp = nullptr;
+      float s = key < k1 ? NAN : -INFINITY;  // a missing page's score is NaN
+      if (page) {
+        const bool fresh = FUSED && key >= it.offset;
+        const int64_t row_at = fresh ? it.q0 + int64_t(key - it.offset) * a.q_r : (key & (g.page_size - 1)) * g.dim;
+        kp = (fresh ? static_cast<const T*>(a.k) : page) + row_at;
+        vp = (fresh ? static_cast<const T*>(a.v) : page + g.kind_stride) + row_at;
+        float sum[E];
+#pragma unroll
+        for (int i = 0; i < E; ++i) sum[i] = 0.f;
+#pragma unroll 1
+        for (int c = 0; c < g.dim; c += E) {
+          float x[E], y[E];
+          const u32x4 qx = *global_view(reinterpret_cast<const u32x4*>(qrow + c));
+          const u32x4 kx = *global_view(reinterpret_cast<const u32x4*>(kp + c));
+          unpack16<DT>(qx, x);
+          unpack16<DT>(kx, y);
+#pragma unroll
+          for (int i = 0; i < E; ++i) sum[i] = fmaf(x[i], y[i], sum[i]);
+        }
+#pragma unroll
+        for (int w = E / 2; w > 0; w /= 2)
+#pragma unroll
+          for (int i = 0; i < w; ++i) sum[i] += sum[i + w];
+        s = sum[0] * a.qscale;
+      }
+      float top = s;
+#pragma unroll
+      for (int w = kWave / 2; w > 0; w /= 2) top = fmaxf(top, __shfl_xor(top, w));
+      top = fmaxf(m, top);
+      const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - top);
+      const float p = fast_exp2(s - (top == -INFINITY ? 0.f : top));
+      m = top;
+      l = fmaf(l, alpha, p);  // this lane's keys
+#pragma unroll
+      for (int e = 0; e < COLS; ++e) acc[e] *= alpha;
+      const uint64_t v_at = reinterpret_cast<uintptr_t>(vp);
+#pragma unroll 4
+      for (int j = 0; j < min(kWave, k1 - k0); ++j) {
+        const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), j));
+        const T* vj = reinterpret_cast<const T*>(
+            uint64_t(uint32_t(__builtin_amdgcn_readlane(int(v_at >> 32), j))) << 32 |
+            uint32_t(__builtin_amdgcn_readlane(int(v_at), j)));
+#pragma unroll
+        for (int e = 0; e < COLS; ++e)
+          if (vj && lane + kWave * e < g.dim)
+            acc[e] = fmaf(pj, to_f32<DT>(global_view(vj)[lane + kWave * e]), acc[e]);
+      }
+    }
+#pragma unroll
+    for (int w = kWave / 2; w > 0; w /= 2) l += __shfl_xor(l, w);
+    float* const part =
+        it.slot >= 0 ? a.partials + ((int64_t(it.slot) * g.heads + it.head) * TQ + q) * pf_part_row<DP>() : nullptr;
+#pragma unroll
+    for (int e = 0; e < COLS; ++e) {
+      const int c = lane + kWave * e;
+      if (part) part[c] = acc[e];
+      else if (c < g.dim) static_cast<T*>(a.out)[it.o0 + row * a.o_r + c] = from_f32<DT>(finalize(acc[e], l));
+    }
+    if (part && lane == 0) *reinterpret_cast<float2*>(part + DP) = float2{m, l};
+  }
+}
+
 template <int DT, int DP, int QT, int KG, int SW, class Items, bool FUSED>
 __global__ __launch_bounds__(QT * KG * kWave) __attribute__((amdgpu_waves_per_eu(SW)))
 void causal_kernel(QueryArgs a, Items items) {
@@ -1550,6 +1652,7 @@ void causal_kernel(QueryArgs a, Items items) {
   constexpr int QW = DT == kF32 ? DP / 8 : DP / 16;  // 16-byte query registers
   __shared__ const T* s_page[kPfWindowPages];
   __shared__ int s_missing;  // whether a page of a window was missing
+  __shared__ uint32_t s_redo[QT];  // queries of the tile to attend alone, a bit each
   __shared__ __align__(16) char s_raw[S::kLds];
   const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)s_raw));
 
@@ -1672,6 +1775,7 @@ void causal_kernel(QueryArgs a, Items items) {
       const int w1 = w0 + win_keys < kstop ? w0 + win_keys : kstop;
       const int npg = (w1 - w0 + g.page_size - 1) >> g.log2_page;
       __syncthreads();  // every wave is done with the LDS of the window before
+      if (KG > 1 && tid < QT) s_redo[tid] = 0;
       // The first round is staged before the window's pages are known when it
       // holds only the prompt's own rows, and again if one turns out missing.
       const bool early = FUSED && w0 >= offset;
@@ -1861,13 +1965,22 @@ void causal_kernel(QueryArgs a, Items items) {
     l = add_halves(l);
     float* const part = it.slot >= 0 ? a.partials + (int64_t(it.slot) * g.heads + head) * TQ * pf_part_row<DP>() : nullptr;
     if constexpr (KG == 1) {
+      // Queries left non-finite (and not by a missing page, whose NaN is the
+      // denominator's too) are attended once more, alone.
+      float zero = 0.f;
+#pragma unroll
+      for (int d = 0; d < DT32; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) zero = fmaf(o[d][i], 0.f, zero);
+      const uint64_t lanes = __ballot(q_ok && isnan(zero) && !isnan(l));
+      const uint32_t redo = uint32_t(lanes) | uint32_t(lanes >> 32);
       const float inv = inverse(l);
 #pragma unroll
       for (int d = 0; d < DT32; ++d)
 #pragma unroll
         for (int i = 0; i < 16; i += 4) {
           const int dd = 32 * d + 2 * i + 4 * grp;
-          if (!q_ok) continue;
+          if (!q_ok || (redo >> col & 1)) continue;
           if (part)
             *reinterpret_cast<float4*>(part + (qt * 32 + col) * pf_part_row<DP>() + dd) =
                 float4{o[d][i], o[d][i + 1], o[d][i + 2], o[d][i + 3]};
@@ -1875,8 +1988,9 @@ void causal_kernel(QueryArgs a, Items items) {
             store4<DT>(out + it.o0 + qi * a.o_r + dd, divided<DT>(o[d][i], l, inv), divided<DT>(o[d][i + 1], l, inv),
                        divided<DT>(o[d][i + 2], l, inv), divided<DT>(o[d][i + 3], l, inv));
         }
-      if (part && q_ok && grp == 0)
+      if (part && q_ok && grp == 0 && !(redo >> col & 1))
         *reinterpret_cast<float2*>(part + (qt * 32 + col) * pf_part_row<DP>() + DP) = float2{m, l};
+      if (redo) attend_again<DT, DP, TQ, 1, Items, FUSED>(item, qt, 0, redo);
     } else {
       // The groups' states meet in LDS, then every thread merges four dims of
       // a query over the groups. A group none of whose keys a query attends
@@ -1894,7 +2008,9 @@ void causal_kernel(QueryArgs a, Items items) {
         if (grp == 0) s_ml[kg * TQ + qt * 32 + col] = float2{m, l};
       }
       __syncthreads();
-      for (int u = tid; u < TQ * DP / 4; u += NT) {
+      int first = tid;
+      asm volatile("" : "+v"(first));  // keeps the addresses below out of the registers of the loop
+      for (int u = first; u < TQ * DP / 4; u += NT) {
         const int q = u / (DP / 4), dd = 4 * (u - q * (DP / 4));
         const int row = it.tile * TQ + q;
         if (row >= nq) break;
@@ -1911,6 +2027,9 @@ void causal_kernel(QueryArgs a, Items items) {
           acc.x = fmaf(x.x, w, acc.x); acc.y = fmaf(x.y, w, acc.y);
           acc.z = fmaf(x.z, w, acc.z); acc.w = fmaf(x.w, w, acc.w);
         }
+        // left non-finite, and not by a missing page: attended once more, alone
+        if (isnan(0.f * acc.x + 0.f * acc.y + 0.f * acc.z + 0.f * acc.w) && !isnan(L))
+          atomicOr(&s_redo[q >> 5], 1u << (q & 31));
         if (part) {
           float* dst = part + q * pf_part_row<DP>();
           *reinterpret_cast<float4*>(dst + dd) = acc;
@@ -1920,6 +2039,13 @@ void causal_kernel(QueryArgs a, Items items) {
           store4<DT>(out + it.o0 + row * a.o_r + dd, divided<DT>(acc.x, L, inv), divided<DT>(acc.y, L, inv),
                      divided<DT>(acc.z, L, inv), divided<DT>(acc.w, L, inv));
         }
+      }
+      // (a workgroup's stores to a row are in the order of its barriers)
+      __syncthreads();
+#pragma unroll 1
+      for (int t = 0; t < QT; ++t) {
+        const uint32_t redo = __builtin_amdgcn_readfirstlane(s_redo[t]);
+        if (redo) attend_again<DT, DP, TQ, S::W, Items, FUSED>(item, t, wave, redo);
       }
     }
   }
