@@ -1468,6 +1468,11 @@ struct CausalShape {
   static constexpr int RW = kWave / CPR;       // rows one load instruction of a wave fills
   static constexpr int DT32 = DP / 32;
   static constexpr int OS = DP + 4;      // row stride of the groups' accumulators in LDS
+  // Parts of a block's keys that an fp32 output sums on its own, four chains
+  // each. Two in the shape for one key block, whose output is one chain's
+  // (60 tokens, head dim 64: 1.040e-7 with one, 1.035e-7 with two, 1.031e-7 in
+  // query_kernel).
+  static constexpr int kSums = DP == 64 && KG == 1 ? 2 : 1;
   static constexpr int kPlane = KI * DP * ES;  // bytes of a round's K (and V)
   // Rounds of LDS: one computed, the others in flight.
   static constexpr int kRing = SW == 4 || KG <= 2 ? 2 : 131072 / (2 * kPlane) < 4 ? 131072 / (2 * kPlane) : 4;
@@ -1910,30 +1915,49 @@ void causal_kernel(QueryArgs a, Items items) {
           m = mn;
         }
         const float mref = (m == -INFINITY) ? 0.f : m;  // masked scores give exp2(-inf) = 0
-        float psum[2] = {0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          sc[i] = fast_exp2(fmaf(sc[i], a.qscale, -mref));
-          psum[i & 1] += sc[i];
-        }
-        l += psum[0] + psum[1];  // this lane's keys; the lanes of a query are added at the end
+        for (int i = 0; i < 16; ++i) sc[i] = fast_exp2(fmaf(sc[i], a.qscale, -mref));
+        float psum[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) psum[i] = sc[i] + sc[i + 8];
+#pragma unroll
+        for (int w = 4; w > 0; w /= 2)
+#pragma unroll
+          for (int i = 0; i < w; ++i) psum[i] += psum[i + w];
+        l += psum[0];  // this lane's keys; the lanes of a query are added at the end
 
         if constexpr (DT == kF32) {
-          // The block's sums start at zero and are added to the running ones,
-          // so that no chain of sums is longer than a block or the blocks.
+          // The block's sums start at zero, in short chains that are added in
+          // pairs and then to the running ones: a chain rounds at every key.
+          // All 32 keys in one chain, 4 x 333 tokens of head dim 64 end 1.38e-7
+          // from 64 bits (2-norm, relative), where query_kernel's short chains
+          // end 1.25e-7; four chains end 1.25e-7 as well, for 2 % of the time
+          // (13 % at head dim 128, one wave per SIMD).
+          constexpr int STEP = 16 / S::kSums;
 #pragma unroll
           for (int d = 0; d < DT32; ++d) {
-            floatx16 ob;
+            floatx16 sum;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ob[i] = 0.f;
+            for (int h = 0; h < 16; h += STEP) {
+              floatx16 ob[4];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int rr = 8 * (i >> 2) + 4 * grp + (i & 3), dd = 32 * d + col;
-              const float vv = s_v[(kg * KB + rr) * DP + S::vpos(rr, dd >> 2) * 4 + (dd & 3)];
-              ob = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, sc[i], ob, 0, 0, 0);
+              for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) ob[j][i] = 0.f;
+#pragma unroll
+              for (int i = h; i < h + STEP; ++i) {
+                const int rr = 8 * (i >> 2) + 4 * grp + (i & 3), dd = 32 * d + col;
+                const float vv = s_v[(kg * KB + rr) * DP + S::vpos(rr, dd >> 2) * 4 + (dd & 3)];
+                ob[i & 3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, sc[i], ob[i & 3], 0, 0, 0);
+              }
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                const float x = (ob[0][i] + ob[1][i]) + (ob[2][i] + ob[3][i]);
+                sum[i] = h ? sum[i] + x : x;
+              }
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) o[d][i] += ob[i];
+            for (int i = 0; i < 16; ++i) o[d][i] += sum[i];
           }
         } else {
           // 16 keys a step: slot j < 4 of a lane holds key 16 s + 4 grp + j,

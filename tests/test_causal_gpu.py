@@ -3,6 +3,7 @@ of its dispatch, against the float64 oracle: head dims that do not fill the
 kernel's 64 or 128 columns, fp32, query counts around the 32-, 64- and
 128-query tiles, every workgroup shape and keys split over workgroups.
 Tolerances are in tests/tolerances.py."""
+import numpy as np
 import pytest
 
 from test_prefill_gpu import prefill_case, run_prefill, run_fused_single, run_ragged
@@ -45,3 +46,16 @@ def test_causal_keys_split_over_workgroups(dtype, dim, nq, offset):
 @pytest.mark.parametrize('dtype,dim', [('float32', 64), ('bfloat16', 80)])
 def test_causal_ragged_splits_over_workgroups(dtype, dim):
     run_ragged(dtype, dim, [1, 33, 20], [2600, 17, 2100], h=2, seed=dim)
+
+
+# Largest relative 2-norm error against 64 bits: 3 % over what the per-query
+# kernel measured on such inputs (1.031e-7, 1.253e-7, 1.436e-7), whose sums are
+# short chains over 16 groups of lanes. One chain over a block's 32 keys gave
+# 1.137e-7, 1.382e-7 and 1.541e-7.
+@pytest.mark.parametrize('dim,n,bound', [(64, 60, 1.06e-7), (64, 333, 1.29e-7), (128, 333, 1.48e-7)])
+def test_fp32_sums_keep_the_per_query_kernels_precision(dim, n, bound):
+    case = prefill_case(700 + n, batch=4, heads=12, dim=dim, page_size=16, nk=n, dtype='float32')
+    got, ref = run_prefill(case, n, n, 0, seed=n)
+    error = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print(f'head dim {dim}, {n} tokens: relative error {error:.4e}')
+    assert error < bound
