@@ -1322,9 +1322,14 @@ struct AppendArgs {
 // The running reference of the exponentials moves only when a score exceeds
 // it by kRescale (base 2), so most blocks skip the rescaling of O: weights
 // are then at most 2^kRescale, which neither fp32 nor the hi/lo split minds.
+// fp16 has nothing below 2^-24, so its weights are taken 2^kHalfShift larger,
+// denominator and all: the split then keeps a weight's 22 bits down to 2^-11 of
+// the largest and ends at 2^-33 of it. At 2^-24, 1500 keys of weight 2^-18
+// beside one of weight 1 lost 1.4 % of their sum.
 constexpr int kPfWindowPages = 512;  // page bases resolved into LDS at a time
 constexpr int kPfBlock = 64;         // keys per unit of a split over workgroups
 constexpr float kRescale = 6.f;
+constexpr float kHalfShift = 9.f;  // 2^(kRescale + kHalfShift) is below fp16's largest
 constexpr int kPfMinQueries = 2;     // a single query runs the decode kernel or query_kernel
 
 // x of lanes l and l ^ 32 (in either order): the permlane swap of two copies
@@ -1655,6 +1660,7 @@ void causal_kernel(QueryArgs a, Items items) {
   constexpr int EC = S::EC, CPR = S::CPR, KB = S::KB, KI = S::KI, NT = S::NT, NC = S::NC, DT32 = S::DT32;
   constexpr int TQ = 32 * QT;
   constexpr int QW = DT == kF32 ? DP / 8 : DP / 16;  // 16-byte query registers
+  constexpr float kShift = DT == kF16 ? kHalfShift : 0.f;
   __shared__ const T* s_page[kPfWindowPages];
   __shared__ int s_missing;  // whether a page of a window was missing
   __shared__ uint32_t s_redo[QT];  // queries of the tile to attend alone, a bit each
@@ -1914,7 +1920,7 @@ void causal_kernel(QueryArgs a, Items items) {
             for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
           m = mn;
         }
-        const float mref = (m == -INFINITY) ? 0.f : m;  // masked scores give exp2(-inf) = 0
+        const float mref = (m == -INFINITY) ? 0.f : m - kShift;  // masked scores give exp2(-inf) = 0
 #pragma unroll
         for (int i = 0; i < 16; ++i) sc[i] = fast_exp2(fmaf(sc[i], a.qscale, -mref));
         float psum[8];
@@ -1987,6 +1993,7 @@ void causal_kernel(QueryArgs a, Items items) {
     // piece of the tile's keys leaves (accumulators, max, denominator) in
     // base-2 units for the merge kernels, a whole tile the output rows.
     l = add_halves(l);
+    m -= kShift;  // what the sums are relative to
     float* const part = it.slot >= 0 ? a.partials + (int64_t(it.slot) * g.heads + head) * TQ * pf_part_row<DP>() : nullptr;
     if constexpr (KG == 1) {
       // Queries left non-finite (and not by a missing page, whose NaN is the

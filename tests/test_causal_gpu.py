@@ -6,7 +6,8 @@ Tolerances are in tests/tolerances.py."""
 import numpy as np
 import pytest
 
-from test_prefill_gpu import prefill_case, run_prefill, run_fused_single, run_ragged
+from oracle import paged_oracle as po
+from test_prefill_gpu import CODES, prefill_case, run_prefill, run_fused_single, run_ragged
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +60,23 @@ def test_fp32_sums_keep_the_per_query_kernels_precision(dim, n, bound):
     error = np.linalg.norm(got - ref) / np.linalg.norm(ref)
     print(f'head dim {dim}, {n} tokens: relative error {error:.4e}')
     assert error < bound
+
+
+@pytest.mark.parametrize('dtype', ['float16', 'bfloat16'])
+@pytest.mark.parametrize('n', [2, 5, 40])
+def test_many_small_weights_beside_large_ones(dtype, n):
+    # In every block of 32 keys one scores 0, with zero values, and 31 score
+    # about -12.75: weights of 2.9e-6, 48.7 of fp16's smallest steps, times
+    # values of 30000 make the whole output, 2.7. Rounded down to whole steps
+    # the weights lost 1 % of it, ten times the tolerance.
+    nk = 1500
+    case = prefill_case(800 + n, batch=1, heads=1, dim=64, page_size=16, nk=nk, dtype=dtype)
+    q = np.random.default_rng(n).standard_normal((1, 1, n, 64), dtype=np.float32)  # as run_prefill draws it
+    q = po.decode(po.encode(q, CODES[dtype]), CODES[dtype])[0, 0].astype(np.float64)
+    k = np.zeros((1, 1, nk, 64), np.float32)
+    k[0, 0] = np.linalg.pinv(q) @ np.full(n, -12.75 * 8)
+    v = np.full_like(k, 30000)
+    k[0, 0, ::32] = v[0, 0, ::32] = 0
+    po.image_append(case.image, case.table, case.columns, po.encode(k, CODES[dtype]), po.encode(v, CODES[dtype]), 0)
+    got, ref = run_prefill(case, n, nk, nk - n, seed=n)
+    assert 2 < ref[0, 0, 0, 0] < 4
