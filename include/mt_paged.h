@@ -161,7 +161,8 @@ int mt_paged_decode_split(void* out, const void* q, const void* k, const void* v
  * 0 = h*d) and out is [b, n, out_stride] with heads merged the same way
  * (0 = h*d). The matrix-core kernel serves n >= 2 with rows of whole 16-byte
  * chunks (d a multiple of 8 in fp16/bf16, of 4 in fp32) at 16-byte aligned
- * addresses. No reference counterpart as one entry (reference
+ * addresses, but for launches of few queries that a walk over the keys per
+ * query ends sooner (d 64 and 128). No reference counterpart as one entry (reference
  * paged_kv_cache.py:205-221 calls mt_paged_append and mt_paged_attention on
  * head-split copies). */
 int mt_paged_prefill(void* out, const void* q, const void* k, const void* v, const uint64_t* slabs,

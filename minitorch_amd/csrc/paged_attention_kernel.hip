@@ -2656,15 +2656,61 @@ hipError_t launch_append(AppendArgs& a, int dtype) {
   return hipGetLastError();
 }
 
+// Whether query_kernel is the faster one for rows that both take (head dims 64
+// and 128, where it reads rows in full 16-byte loads). It walks the keys once
+// per query, four queries of a head side by side; the causal kernel computes
+// tiles of 32 queries however few there are, and fp32 products at a sixteenth
+// of the 16-bit rate. us per call of attention, causal kernel and query_kernel,
+// 12 heads:
+// * fp32, up to four queries: one walk serves them all. 2 queries of 64 requests
+//   at 500 keys 122 and 50, of one request at 60 keys 10.2 and 6.3. Past 512
+//   keys only where the requests fill the compute units (head dim 128: half of
+//   them, its tiles split their keys two ways only): 24 requests at 800 keys 52
+//   and 30, but 16 at 1500 47 and 56; past 1024 for three (64 requests at 1500
+//   keys: 147 in narrow tiles, 139 and 162 for three and four).
+// * fp32, head dim 128, up to eight where the tiles come to between one and two
+//   rounds of the compute units: 32 requests at 500 keys 98 and 91.
+// * fp32, any number of queries while their walks take one round of the compute
+//   units and are short: 64 tokens 9.9 and 6.5, 20 at 120 keys 11.4 and 9.4 (head
+//   dim 128: 23 and 14; 8 at 500 keys 33 and 26). A walk of 16 keys a step ends
+//   later from 256 keys on (384 at head dim 128, 512 for twelve queries).
+// * fp16 and bf16, head dim 64, up to three queries (four to 512 keys) of
+//   requests for more than two rounds: 2 of 64 requests at 500 keys 26 and 20,
+//   of 32 requests 14 and 18. Head dim 128: between one and two rounds to 320
+//   keys, 2 of 32 requests at 200 keys 20 and 15.
+bool query_kernel_faster(const QueryArgs& a, int dtype) {
+  const int d = a.g.dim;
+  if (d != 64 && d != 128) return false;
+  const bool wide = d == 128;
+  const int64_t cus = std::max(1, device_compute_units());
+  const int64_t bh = int64_t(a.batch) * a.g.heads;
+  const int64_t tiles = bh * ((a.nq + 31) / 32), groups = bh * ((a.nq + kWaves - 1) / kWaves);
+  const int keys = a.nk;
+  const bool second_round = tiles > cus && tiles <= 2 * cus;
+  if (dtype != kF32) {
+    if (wide) return a.nq <= 3 && second_round && keys > 128 && keys <= 320;
+    return (a.nq <= 3 || (a.nq == 4 && keys <= 512)) && tiles > 2 * cus && keys > 128;
+  }
+  if (a.nq <= 4 && keys > 32) {
+    if (keys <= 512) return true;
+    if (wide ? 2 * tiles > cus : tiles > cus && (a.nq <= 3 || keys <= 1024)) return true;
+  }
+  if (wide && a.nq <= 8 && second_round && keys > 64) return true;
+  if (keys <= 64) return groups <= (wide ? cus : 2 * cus);
+  return groups <= cus && keys <= (wide ? (a.nq <= 12 ? 512 : 384) : 256);
+}
+
 // Whether launch_query runs the matrix-core causal kernel: rows of whole
 // 16-byte chunks (head dims 8, 16, .. 128 in fp16/bf16, 4, 8, .. in fp32) at
-// 16-byte aligned addresses and at least kPfMinQueries queries.
+// 16-byte aligned addresses and at least kPfMinQueries queries, where
+// query_kernel is not the faster one.
 bool causal_kernel_takes(const QueryArgs& a, int dtype) {
   const int d = a.g.dim;
   const int esize = dtype == kF32 ? 4 : 2;
   auto rows16 = [&](int64_t x) { return (x * esize) % 16 == 0; };
   return rows16(d) && a.nq >= kPfMinQueries && aligned16(a.out) && aligned16(a.q) && rows16(a.q_b) &&
-         rows16(a.q_h) && rows16(a.q_r) && rows16(a.o_b) && rows16(a.o_h) && rows16(a.o_r);
+         rows16(a.q_h) && rows16(a.q_r) && rows16(a.o_b) && rows16(a.o_h) && rows16(a.o_r) &&
+         !query_kernel_faster(a, dtype);
 }
 
 // Launches that split long prompts' keys (a diagnostic for tests).
@@ -2690,7 +2736,7 @@ struct CausalPlan {
 
 // tiles32/64/128: workgroups (tiles x heads, over all prompts) for tiles of
 // that many queries; blocks: key blocks of the longest tile; row_bytes: a K
-// row in LDS. Where the lines lie (MI355X, 256 compute units, us per call):
+// row in LDS; queries: of the longest prompt. Where the lines lie (MI355X, 256 compute units, us per call):
 // * kTiny and kShort for prompts of one and two key blocks, which end before
 //   wider workgroups have met: 8 x 100 tokens x 25 heads fp16 9.3 kShort
 //   against 11.5 kDense.
@@ -2698,6 +2744,11 @@ struct CausalPlan {
 //   eighth more still end with the long tiles): 300 tokens x 12 heads bf16 8.0
 //   against 8.8 kDeep, 700 x 12 fp32 (264 workgroups) 25.8 against 33.1; but
 //   1000 x 16 bf16 (512) 17.5 against 15.2 kDeep.
+//   Also for every launch of prompts of at most 32 queries in rows of more than
+//   128 bytes: half the waves of a wider tile would have none (fp32, 8 queries
+//   of 64 requests at 500 keys x 12 heads 62 against 120 kDeep, head dim 128 177
+//   against 247). Shorter rows keep kDense, whose second workgroup per compute
+//   unit makes up for it (fp16: 26 against 28).
 // * kDeep while 64-query tiles take one round; then kDense, whose second
 //   workgroup per compute unit covers for the first: 1000 x 25 bf16 18.9
 //   against 21.5 kDeep and 24.8 kWide.
@@ -2708,10 +2759,16 @@ struct CausalPlan {
 //   narrow tiles leave half the compute units idle and the longest walks at
 //   least 8 rounds, in pieces of at least 3 (40 tokens at offset 4000 x 12
 //   heads bf16: 15.5 against 26.9).
-CausalPlan causal_plan(int64_t tiles32, int64_t tiles64, int64_t tiles128, int blocks, int row_bytes) {
+CausalPlan causal_plan(int64_t tiles32, int64_t tiles64, int64_t tiles128, int blocks, int row_bytes, int queries) {
   const int64_t cus = std::max(1, device_compute_units());
   CausalPlan plan{};
-  plan.config = blocks == 1 ? kTiny : blocks == 2 ? kShort : 8 * tiles32 <= 9 * cus ? kNarrow : tiles64 <= cus ? kDeep : 2 * tiles128 < 3 * cus ? kDense : kWide;
+  const bool narrow = 8 * tiles32 <= 9 * cus || (queries <= 32 && row_bytes > 128);
+  plan.config = blocks == 1             ? kTiny
+                : blocks == 2           ? kShort
+                : narrow                ? kNarrow
+                : tiles64 <= cus        ? kDeep
+                : 2 * tiles128 < 3 * cus ? kDense
+                                        : kWide;
   const int round = std::max(1, 4 * 128 / row_bytes);  // blocks a narrow workgroup takes per round
   if (plan.config == kNarrow && 2 * tiles32 <= cus && blocks >= 8 * round) {
     const int64_t pieces = std::min<int64_t>(std::min<int64_t>(cus / tiles32, 64), blocks / (3 * round));
@@ -2787,7 +2844,7 @@ hipError_t launch_query(QueryArgs& a, int dtype) {
     auto tiles = [&](int tq) { return (a.nq + tq - 1) / tq; };
     const int most = key_blocks(tiles(64) - 1, 64, a.nq, a.offset);
     const CausalPlan plan = causal_plan(bh * tiles(32), bh * tiles(64), bh * tiles(128), most,
-                                         (d <= 64 ? 64 : 128) * esize);
+                                         (d <= 64 ? 64 : 128) * esize, a.nq);
     const int tq = config_queries(plan.config);
     UniformItems items{tiles(tq), 1, 0};
     if (plan.share > 0) {
@@ -2961,6 +3018,7 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
     int r1 = r0;
     int64_t rows = 0;
     int most = 0;  // key blocks of the longest tile
+    int queries = 0;  // tokens of the longest prompt
     int64_t tiles32 = 0, tiles64 = 0, tiles128 = 0, total_blocks = 0;
     while (r1 < requests && r1 - r0 < kRaggedPrompts && tiles64 + (tokens[r1] + 63) / 64 <= kRaggedTiles) {
       const int p = r1 - r0;
@@ -2968,6 +3026,7 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
       it.n[p] = tokens[r1];
       it.offset[p] = offsets[r1];
       it.table[p] = tables[r1];
+      queries = std::max(queries, tokens[r1]);
       most = std::max(most, key_blocks((tokens[r1] - 1) / 64, 64, tokens[r1], offsets[r1]));
       for (int t = 0; t * 64 < tokens[r1]; ++t) total_blocks += key_blocks(t, 64, tokens[r1], offsets[r1]);
       tiles32 += (tokens[r1] + 31) / 32;
@@ -2992,7 +3051,8 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
     it.prompts = r1 - r0;
     // (narrow tiles only where the launch can list them)
     const CausalPlan plan = causal_plan(tiles32 <= kRaggedTiles ? tiles32 * h : INT64_MAX / 16, tiles64 * h,
-                                        tiles128 * h, most, (d <= 64 ? 64 : 128) * int(e));
+                                        tiles128 * h, most, (d <= 64 ? 64 : 128) * int(e),
+                                        tiles32 <= kRaggedTiles ? queries : INT_MAX);
     const int tq = config_queries(plan.config);
     // (prompt, tile) pairs and their key blocks, the longest first; with a
     // share, cut into pieces of at most that many blocks as far as the

@@ -32,6 +32,23 @@ def test_causal_workgroup_shapes(dtype, batch, heads, nq, offset):
     run_prefill(case, nq, offset + nq, offset, seed=heads)
 
 
+# (batch, heads, queries, offset, head dim) about the lines between the causal
+# and the per-query kernel, and of prompts of at most 32 queries over one round
+# of the compute units, whose tiles are narrow: fp32 in grids that the causal
+# kernel takes at few queries or keys, then few queries on the per-query kernel
+@pytest.mark.parametrize('dtype,shape', [
+    ('float32', (8, 70, 2, 10, 64)), ('float32', (4, 20, 31, 33, 64)), ('float32', (4, 20, 33, 0, 64)),
+    ('float32', (3, 30, 65, 31, 64)), ('float32', (5, 52, 20, 300, 64)), ('float32', (6, 50, 20, 300, 64)),
+    ('float32', (6, 50, 20, 300, 128)), ('float32', (4, 140, 7, 150, 128)), ('bfloat16', (6, 50, 20, 300, 80)),
+    ('float32', (30, 10, 4, 508, 64)), ('float32', (30, 10, 4, 1021, 64)), ('float32', (30, 10, 3, 1022, 128)),
+    ('float32', (4, 80, 7, 150, 128)), ('float32', (1, 12, 20, 380, 128)), ('float16', (30, 20, 3, 200, 64)),
+    ('bfloat16', (30, 20, 4, 508, 64)), ('float16', (30, 10, 3, 317, 128)), ('float16', (30, 10, 3, 318, 128))])
+def test_few_queries(dtype, shape):
+    batch, heads, nq, offset, dim = shape
+    case = prefill_case(450 + nq + heads, batch=batch, heads=heads, dim=dim, page_size=16, nk=offset + nq, dtype=dtype)
+    run_prefill(case, nq, offset + nq, offset, seed=heads)
+
+
 @pytest.mark.parametrize('dtype,dim', [('float32', 64), ('bfloat16', 64), ('float16', 80)])
 @pytest.mark.parametrize('nq,offset', [(3, 4090), (40, 2500)])
 def test_causal_keys_split_over_workgroups(dtype, dim, nq, offset):
