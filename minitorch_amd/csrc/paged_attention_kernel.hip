@@ -1998,12 +1998,12 @@ void causal_kernel(QueryArgs a, Items items) {
     if constexpr (KG == 1) {
       // Queries left non-finite (and not by a missing page, whose NaN is the
       // denominator's too) are attended once more, alone.
-      float zero = 0.f;
+      float zero[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int d = 0; d < DT32; ++d)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) zero = fmaf(o[d][i], 0.f, zero);
-      const uint64_t lanes = __ballot(q_ok && isnan(zero) && !isnan(l));
+        for (int i = 0; i < 16; ++i) zero[i & 3] = fmaf(o[d][i], 0.f, zero[i & 3]);
+      const uint64_t lanes = __ballot(q_ok && isnan((zero[0] + zero[1]) + (zero[2] + zero[3])) && !isnan(l));
       const uint32_t redo = uint32_t(lanes) | uint32_t(lanes >> 32);
       const float inv = inverse(l);
 #pragma unroll
@@ -2011,7 +2011,7 @@ void causal_kernel(QueryArgs a, Items items) {
 #pragma unroll
         for (int i = 0; i < 16; i += 4) {
           const int dd = 32 * d + 2 * i + 4 * grp;
-          if (!q_ok || (redo >> col & 1)) continue;
+          if (!q_ok) continue;
           if (part)
             *reinterpret_cast<float4*>(part + (qt * 32 + col) * pf_part_row<DP>() + dd) =
                 float4{o[d][i], o[d][i + 1], o[d][i + 2], o[d][i + 3]};
@@ -2019,9 +2019,12 @@ void causal_kernel(QueryArgs a, Items items) {
             store4<DT>(out + it.o0 + qi * a.o_r + dd, divided<DT>(o[d][i], l, inv), divided<DT>(o[d][i + 1], l, inv),
                        divided<DT>(o[d][i + 2], l, inv), divided<DT>(o[d][i + 3], l, inv));
         }
-      if (part && q_ok && grp == 0 && !(redo >> col & 1))
+      if (part && q_ok && grp == 0)
         *reinterpret_cast<float2*>(part + (qt * 32 + col) * pf_part_row<DP>() + DP) = float2{m, l};
-      if (redo) attend_again<DT, DP, TQ, 1, Items, FUSED>(item, qt, 0, redo);
+      if (__builtin_expect(redo != 0, 0)) {
+        __threadfence_block();  // after the stores above, which it repeats
+        attend_again<DT, DP, TQ, 1, Items, FUSED>(item, qt, 0, redo);
+      }
     } else {
       // The groups' states meet in LDS, then every thread merges four dims of
       // a query over the groups. A group none of whose keys a query attends
@@ -2059,7 +2062,7 @@ void causal_kernel(QueryArgs a, Items items) {
           acc.z = fmaf(x.z, w, acc.z); acc.w = fmaf(x.w, w, acc.w);
         }
         // left non-finite, and not by a missing page: attended once more, alone
-        if (isnan(0.f * acc.x + 0.f * acc.y + 0.f * acc.z + 0.f * acc.w) && !isnan(L))
+        if (__builtin_expect(isnan(0.f * acc.x + 0.f * acc.y + 0.f * acc.z + 0.f * acc.w) && !isnan(L), 0))
           atomicOr(&s_redo[q >> 5], 1u << (q & 31));
         if (part) {
           float* dst = part + q * pf_part_row<DP>();
@@ -2073,11 +2076,13 @@ void causal_kernel(QueryArgs a, Items items) {
       }
       // (a workgroup's stores to a row are in the order of its barriers)
       __syncthreads();
+      uint32_t any = 0;
+#pragma unroll
+      for (int t = 0; t < QT; ++t) any |= s_redo[t];
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) != 0, 0))
 #pragma unroll 1
-      for (int t = 0; t < QT; ++t) {
-        const uint32_t redo = __builtin_amdgcn_readfirstlane(s_redo[t]);
-        if (redo) attend_again<DT, DP, TQ, S::W, Items, FUSED>(item, t, wave, redo);
-      }
+        for (int t = 0; t < QT; ++t)
+          attend_again<DT, DP, TQ, S::W, Items, FUSED>(item, t, wave, __builtin_amdgcn_readfirstlane(s_redo[t]));
     }
   }
 }
