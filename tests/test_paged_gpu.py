@@ -444,3 +444,20 @@ def test_many_residency_rounds_back_to_back():
     for _ in range(7):
         again = run_decode(dev)
         assert np.array_equal(first.view(np.uint16), again.view(np.uint16))
+
+
+def test_fp32_row_of_many_splits_keeps_its_precision():
+    # One row of 8000 tokens x 12 heads, 63 splits where the library chooses.
+    # Relative 2-norm errors against 64 bits, mean of four draws: 1.87e-7 with
+    # the splits' terms added in pairs, 2.17e-7 in one chain, 1.96e-7 in the 8
+    # splits of 1024 tokens.
+    errors = []
+    for seed in range(4):
+        case = make_decode_case(610 + seed, batch=1, heads=12, dim=64, page_size=16, lengths=[8000],
+                                pool_pages=512, pages_per_slab=64, dtype='float32')
+        ref = po.image_decode_batch(case.image.copy(), po.F32, case.table, case.columns, case.q, case.k, case.v,
+                                    case.offsets, case.layer)
+        got = run_decode(DevicePagedCase(case))
+        errors.append(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+    print('relative errors', ['%.3e' % e for e in errors])
+    assert np.mean(errors) < 2.0e-7
