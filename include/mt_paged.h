@@ -55,7 +55,10 @@ int mt_paged_attention(void* out, const void* q, const uint64_t* slabs, const in
  * host threads, each on its own default stream, never share one -- kept
  * until the thread exits and grown stream-ordered on the calling thread's
  * default stream (hipMallocAsync / hipFreeAsync, no device synchronization)
- * when a table needs more; status 2 if it cannot grow. Batches of at most
+ * when a table needs more; status 2 if it cannot grow. A graph captured with
+ * this call (or with another that splits keys) holds the workspace's address,
+ * which stays valid while the capturing thread lives; its replays and the
+ * thread's other calls belong on that thread's stream. Batches of at most
  * 256 rows with tables of at most 1024 tokens allocate nothing.
  * Replaces reference mt_paged_decode_batch (src/paged_attention_kernel.cu:121-137). */
 int mt_paged_decode_batch(void* out, const void* q, const void* k, const void* v,

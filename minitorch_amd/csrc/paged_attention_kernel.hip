@@ -2527,52 +2527,79 @@ size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
 // grows stream-ordered on that stream: hipMallocAsync for the larger buffer
 // and hipFreeAsync for the old one, which is released only after the work
 // queued before it, so growing neither synchronizes the device nor blocks the
-// host. A thread's buffers are released (stream-ordered) when it exits.
+// host. A buffer whose address a captured graph holds is not released while
+// its thread lives, nor is one that a capture outgrows, where a release would be
+// a node of the graph; the buffer that takes its place is at least twice as
+// large, so that those kept add up to less than the current one. Under capture
+// the larger buffer is a plain allocation: a stream-ordered one would be a node
+// too, there only while the graph runs. A thread's buffers are released when it
+// exits.
 // Callers that cannot allocate use mt_paged_decode_split with their own
 // workspace, or mt_paged_decode_batch_noalloc.
+struct Workspace {
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  bool pooled = false;    // from hipMallocAsync
+  bool captured = false;  // a graph holds its address
+};
+
 struct ThreadWorkspaces {
-  std::vector<std::pair<void*, size_t>> per_device;
+  struct PerDevice {
+    Workspace current;
+    std::vector<Workspace> kept;
+  };
+  std::vector<PerDevice> per_device;
+  static void release(const Workspace& w) {
+    if (w.ptr) (void)(w.pooled ? hipFreeAsync(w.ptr, hipStreamPerThread) : hipFree(w.ptr));
+  }
   ~ThreadWorkspaces() {
     int current = 0;
     if (hipGetDevice(&current) != hipSuccess) return;
     for (size_t dev = 0; dev < per_device.size(); ++dev) {
-      if (!per_device[dev].first || hipSetDevice(int(dev)) != hipSuccess) continue;
-      (void)hipFreeAsync(per_device[dev].first, hipStreamPerThread);
+      if (!per_device[dev].current.ptr || hipSetDevice(int(dev)) != hipSuccess) continue;
+      release(per_device[dev].current);
+      for (const Workspace& w : per_device[dev].kept) release(w);
     }
     (void)hipSetDevice(current);
   }
 };
 thread_local ThreadWorkspaces t_workspaces;
 
-// `capturing` false: refused while the stream is captured. A buffer grown
-// there would belong to the graph, and a later call that grows the buffer
-// frees the one that the graph's replays would still write to.
-int library_workspace(size_t bytes, void** out, bool capturing = true) {
+int library_workspace(size_t bytes, void** out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  auto& ws = t_workspaces.per_device;
-  if (ws.size() <= size_t(dev)) ws.resize(dev + 1, {nullptr, 0});
-  auto& slot = ws[dev];
-  if (!capturing) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(hipStreamPerThread, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
-      return hipErrorOutOfMemory;
-  }
-  if (slot.second < bytes) {
-    void* p = nullptr;
-    e = hipMallocAsync(&p, bytes, hipStreamPerThread);
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  e = hipStreamIsCapturing(hipStreamPerThread, &status);
+  if (e != hipSuccess) return e;
+  const bool capturing = status != hipStreamCaptureStatusNone;
+  auto& per_device = t_workspaces.per_device;
+  if (per_device.size() <= size_t(dev)) per_device.resize(dev + 1);
+  auto& ws = per_device[dev];
+  if (ws.current.bytes < bytes) {
+    Workspace w;
+    const bool keep = ws.current.ptr && (capturing || ws.current.captured);
+    w.bytes = keep ? std::max(bytes, 2 * ws.current.bytes) : bytes;
+    w.pooled = !capturing;
+    if (capturing) {
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      e = hipThreadExchangeStreamCaptureMode(&mode);
+      if (e != hipSuccess) return e;
+      e = hipMalloc(&w.ptr, w.bytes);
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+    } else {
+      e = hipMallocAsync(&w.ptr, w.bytes, hipStreamPerThread);
+    }
     if (e != hipSuccess) {
       (void)hipGetLastError();  // the caller reports the status; keep it off the next launch
       return e;
     }
-    if (slot.first) {
-      e = hipFreeAsync(slot.first, hipStreamPerThread);
-      if (e != hipSuccess) return e;
-    }
-    slot = {p, bytes};
+    if (keep) ws.kept.push_back(ws.current);
+    else if (ws.current.ptr) (void)hipFreeAsync(ws.current.ptr, hipStreamPerThread);
+    ws.current = w;
   }
-  *out = slot.first;
+  ws.current.captured |= capturing;
+  *out = ws.current.ptr;
   return hipSuccess;
 }
 
@@ -2632,7 +2659,7 @@ hipError_t decode_uniform(void* out, const void* q, const void* k, const void* v
   a.nsplit_max = (len + a.split_tokens - 1) / a.split_tokens;
   if (a.nsplit_max > 1) {
     void* ws = nullptr;
-    if (library_workspace(workspace_bytes_for(bh, a.nsplit_max), &ws, false) != hipSuccess) return hipErrorNotSupported;
+    if (library_workspace(workspace_bytes_for(bh, a.nsplit_max), &ws) != hipSuccess) return hipErrorNotSupported;
     a.partials = static_cast<float*>(ws);
   }
   a.out = out; a.q = q; a.k = k; a.v = v; a.slabs = slabs; a.table = table;
@@ -2864,7 +2891,7 @@ hipError_t launch_query(QueryArgs& a, int dtype) {
       void* ws = nullptr;
       // Without room for the partials the launch runs unsplit.
       if (pieces > 1 && library_workspace(size_t(bh) * items.tiles * pieces * tq * (d <= 64 ? 68 : 132) * sizeof(float),
-                                          &ws, false) == hipSuccess) {
+                                          &ws) == hipSuccess) {
         items.pieces = pieces;
         items.share = plan.share;
         a.partials = static_cast<float*>(ws);
@@ -3100,7 +3127,7 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
       // Without room for the partials the launch runs unsplit.
       pairs = cut(true);
       if (most > 65535 ||
-          (slots && library_workspace(size_t(slots) * h * tq * (d <= 64 ? 68 : 132) * sizeof(float), &ws, false) != hipSuccess)) {
+          (slots && library_workspace(size_t(slots) * h * tq * (d <= 64 ? 68 : 132) * sizeof(float), &ws) != hipSuccess)) {
         share = slots = 0;
         mg = RaggedMerge{};
       }
