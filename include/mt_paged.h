@@ -92,12 +92,10 @@ int mt_paged_decode_batch_noalloc(void* out, const void* q, const void* k, const
                                   int b, int h, int d, int page_size, int pages_per_slab,
                                   int num_slabs, int columns, int layer, int layers, int dtype);
 
-/* Number of launches since the library was loaded in which
- * mt_paged_attention / mt_paged_prefill split one long prompt's keys over
- * wave groups or workgroups because the prompt alone leaves compute units idle
- * (64-query tiles x heads <= compute units, >= 6 key blocks of 64 in the last
- * tile), and of mt_paged_prefill_ragged launches whose longest tile spans at
- * least 6 key blocks and more than its share of the launch. A diagnostic, e.g.
+/* Number of launches of mt_paged_attention, mt_paged_prefill and
+ * mt_paged_prefill_ragged since the library was loaded that split prompts' keys
+ * over workgroups, whose partial results a second launch merged (prompts that
+ * leave half the compute units idle, over long contexts). A diagnostic, e.g.
  * for tests that must exercise that path. No reference counterpart. */
 int mt_paged_prefill_key_splits(long long* launches);
 

@@ -2752,7 +2752,7 @@ bool causal_kernel_takes(const QueryArgs& a, int dtype) {
          !query_kernel_faster(a, dtype);
 }
 
-// Launches that split long prompts' keys (a diagnostic for tests).
+// Launches that split prompts' keys over workgroups (a diagnostic for tests).
 std::atomic<long long> g_key_split_launches{0};
 
 // Workgroup shapes of a causal launch (QT x KG waves, SW): queries per tile
@@ -2814,13 +2814,6 @@ CausalPlan causal_plan(int64_t tiles32, int64_t tiles64, int64_t tiles128, int b
     plan.share = int((blocks + pieces - 1) / pieces);
   }
   return plan;
-}
-
-// Counts a launch that shortened its longest tiles by splitting their keys
-// over wave groups or workgroups: tiles of at least 6 blocks whose prompts
-// alone would not have kept the compute units busy.
-void count_key_split(bool idle, int blocks) {
-  if (idle && blocks >= 6) g_key_split_launches.fetch_add(1, std::memory_order_relaxed);
 }
 
 template <int DT, int DP, class Items, bool FUSED>
@@ -2908,8 +2901,8 @@ hipError_t launch_query(QueryArgs& a, int dtype) {
       else if (dtype == kF16) { MT_MERGE(kF16) }
       else { MT_MERGE(kBF16) }
 #undef MT_MERGE
+      g_key_split_launches.fetch_add(1, std::memory_order_relaxed);
     }
-    count_key_split(a.batch == 1 && bh * tiles(64) <= device_compute_units(), most);
     return hipGetLastError();
   }
   if (a.k) return hipErrorInvalidValue;
@@ -3058,7 +3051,7 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
     int64_t rows = 0;
     int most = 0;  // key blocks of the longest tile
     int queries = 0;  // tokens of the longest prompt
-    int64_t tiles32 = 0, tiles64 = 0, tiles128 = 0, total_blocks = 0;
+    int64_t tiles32 = 0, tiles64 = 0, tiles128 = 0;
     while (r1 < requests && r1 - r0 < kRaggedPrompts && tiles64 + (tokens[r1] + 63) / 64 <= kRaggedTiles) {
       const int p = r1 - r0;
       it.first_row[p] = int(rows);
@@ -3067,7 +3060,6 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
       it.table[p] = tables[r1];
       queries = std::max(queries, tokens[r1]);
       most = std::max(most, key_blocks((tokens[r1] - 1) / 64, 64, tokens[r1], offsets[r1]));
-      for (int t = 0; t * 64 < tokens[r1]; ++t) total_blocks += key_blocks(t, 64, tokens[r1], offsets[r1]);
       tiles32 += (tokens[r1] + 31) / 32;
       tiles64 += (tokens[r1] + 63) / 64;
       tiles128 += (tokens[r1] + 127) / 128;
@@ -3168,11 +3160,10 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
       else if (dtype == kF16) { MT_MERGE(kF16) }
       else { MT_MERGE(kBF16) }
 #undef MT_MERGE
+      g_key_split_launches.fetch_add(1, std::memory_order_relaxed);
     }
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    // the longest tile against its share of the launch over two workgroups per compute unit
-    count_key_split(int64_t(most) * 2 * std::max(1, device_compute_units()) > total_blocks * h, most);
     r0 = r1;
     row0 += rows;
   }

@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 from oracle import paged_oracle as po
-from test_prefill_gpu import CODES, prefill_case, run_prefill, run_fused_single, run_ragged
+from test_prefill_gpu import (CODES, key_split_launches, prefill_case, run_prefill, run_fused_single,
+                              run_ragged)
 
 pytestmark = pytest.mark.gpu
 
@@ -55,15 +56,21 @@ def test_causal_keys_split_over_workgroups(dtype, dim, nq, offset):
     # few tiles, many rounds of keys; a hole is NaN for every query through the merge
     case = prefill_case(500 + nq, batch=1, heads=2, dim=dim, page_size=8, nk=offset + nq, dtype=dtype,
                         pages_per_slab=16)
+    before = key_split_launches()
     run_prefill(case, nq, offset + nq, offset, seed=nq)
+    assert key_split_launches() == before + 1
     run_fused_single(case, nq, offset, seed=nq)
+    assert key_split_launches() == before + 2
     case.table[0, 100] = -1
     run_prefill(case, nq, offset + nq, offset, seed=nq)
+    assert key_split_launches() == before + 3
 
 
 @pytest.mark.parametrize('dtype,dim', [('float32', 64), ('bfloat16', 80)])
 def test_causal_ragged_splits_over_workgroups(dtype, dim):
+    before = key_split_launches()
     run_ragged(dtype, dim, [1, 33, 20], [2600, 17, 2100], h=2, seed=dim)
+    assert key_split_launches() == before + 1
 
 
 # Largest relative 2-norm error against 64 bits: 3 % over what the per-query

@@ -136,9 +136,8 @@ def test_prefill_large_scores(dtype):
     run_prefill(case, nq, nq, 0, seed=8)
 
 
-def test_prefill_matches_per_query_kernel_below_threshold():
-    # 15 and 16 queries (once the two sides of the matrix-core kernel's
-    # threshold) against the oracle on the same pages.
+def test_prefill_fifteen_and_sixteen_queries():
+    # both on the matrix-core kernel, against the oracle on the same pages
     case = prefill_case(47, batch=2, heads=2, dim=64, page_size=16, nk=60, dtype='float16')
     dev = DevicePagedCase(case)
     run_prefill(case, 15, 59, 44, seed=9, dev=dev)
@@ -247,7 +246,7 @@ def test_prefill_ragged_more_prompts_than_one_launch_takes():
     run_ragged('float16', 64, tokens, [int(o) for o in rng.integers(0, 40, 20)], h=2, seed=3)
 
 
-def test_prefill_ragged_fp32_takes_the_per_prompt_path():
+def test_prefill_ragged_fp32():
     run_ragged('float32', 64, [17, 3, 40], [0, 12, 5], h=2, seed=4)
 
 
@@ -338,9 +337,10 @@ def test_fused_append_with_missing_page_equals_append_then_attention(entry):
 @pytest.mark.parametrize('dim', [64, 128])
 @pytest.mark.parametrize('nq,offset,page_size', [(1024, 0, 16), (700, 333, 32), (300, 2000, 8)])
 def test_prefill_long_single_prompt_key_splits(dtype, dim, nq, offset, page_size):
-    # One request of a few heads with a long context: its query tiles leave
-    # most compute units idle, so their keys are split over workgroups and
-    # merged (log-sum-exp). Against the oracle, through both entries: causal
+    # One request of a few heads with a long context, whose query tiles leave
+    # most compute units idle: where it has rounds of keys enough (300 tokens at
+    # offset 2000, and every case of head dim 128) they are split over workgroups
+    # and merged (log-sum-exp). Against the oracle, through both entries: causal
     # attention over appended pages, and the fused append + attention.
     case = prefill_case(80 + nq, batch=1, heads=2, dim=dim, page_size=page_size, nk=offset + nq, dtype=dtype,
                         pages_per_slab=8)
@@ -381,13 +381,15 @@ def run_fused_single(case, n, offset, seed=0):
 def test_prefill_key_splits_with_missing_pages():
     # holes inside the split key range: the queries that attend them are NaN,
     # the others are not (the merge keeps a NaN denominator)
-    nq, offset = 900, 50
+    nq, offset = 900, 1250
     case = prefill_case(91, batch=1, heads=2, dim=64, page_size=16, nk=offset + nq, dtype='bfloat16',
                         pages_per_slab=8)
-    case.table[0, 10] = -1          # keys 160..175
-    case.table[0, 40] = 10 ** 6     # keys 640..655
+    case.table[0, 88] = -1          # keys 1408..1423
+    case.table[0, 118] = 10 ** 6    # keys 1888..1903
+    before = key_split_launches()
     got, ref = run_prefill(case, nq, offset + nq, offset, seed=9)
-    assert np.isnan(ref[0, :, 160 - offset:]).all() and not np.isnan(ref[0, :, :160 - offset]).any()
+    assert key_split_launches() == before + 1
+    assert np.isnan(ref[0, :, 1408 - offset:]).all() and not np.isnan(ref[0, :, :1408 - offset]).any()
 
 
 def key_split_launches():
@@ -402,23 +404,30 @@ def key_split_launches():
 @pytest.mark.parametrize('dtype', ['float16', 'bfloat16'])
 @pytest.mark.parametrize('heads,dim', [(12, 64), (16, 64), (12, 128), (16, 128)])
 def test_prefill_key_split_at_model_head_counts(heads, dim, dtype):
-    # The shapes the split is for: a 1024-token prompt of DistilGPT-2 (12
-    # heads; 16 tiles x 12 heads, B = 4 key blocks per split) and GPT-2-medium
-    # (16 heads; 256 workgroups, an odd B = 5), at head_dim 64 and 128, through
-    # mt_paged_attention (pages) and mt_paged_prefill (fused append); each
-    # must take the key-split path, checked with the library's counter.
+    # 40 tokens of DistilGPT-2 (12 heads) and GPT-2-medium (16 heads) behind a
+    # long context, at head_dim 64 and 128: 24 and 32 narrow tiles of 64 key
+    # blocks, whose keys are split over workgroups and merged, through
+    # mt_paged_attention (pages) and mt_paged_prefill (fused append); each must
+    # take that path, checked with the library's counter. A prompt of 1024
+    # tokens, whose tiles fill the compute units, must not.
+    nq, offset = 40, 4051
+    case = prefill_case(90 + heads + dim, batch=1, heads=heads, dim=dim, page_size=16, nk=offset + nq, dtype=dtype,
+                        pages_per_slab=8)
+    before = key_split_launches()
+    run_prefill(case, nq, offset + nq, offset, seed=heads + dim)
+    assert key_split_launches() == before + 1, 'mt_paged_attention did not split the keys'
+    run_fused_single(case, nq, offset, seed=heads + dim)
+    assert key_split_launches() == before + 2, 'mt_paged_prefill did not split the keys'
     nq = 1024
     case = prefill_case(90 + heads + dim, batch=1, heads=heads, dim=dim, page_size=16, nk=nq, dtype=dtype,
                         pages_per_slab=8)
-    before = key_split_launches()
     run_prefill(case, nq, nq, 0, seed=heads + dim)
-    assert key_split_launches() == before + 1, 'mt_paged_attention did not split the keys'
     run_fused_single(case, nq, 0, seed=heads + dim)
-    assert key_split_launches() == before + 2, 'mt_paged_prefill did not split the keys'
+    assert key_split_launches() == before + 2
 
 
 def test_prefill_above_the_split_limit_stays_unsplit():
-    # 25 heads x 16 query tiles = 400 workgroups > 256 compute units: the
+    # 25 heads x 32 narrow tiles = 800 workgroups > 256 compute units: the
     # prompt already fills the GPU, so it runs unsplit (and still matches)
     nq, heads = 1024, 25
     case = prefill_case(97, batch=1, heads=heads, dim=64, page_size=16, nk=nq, dtype='bfloat16', pages_per_slab=8)
@@ -431,14 +440,17 @@ def test_prefill_above_the_split_limit_stays_unsplit():
 @pytest.mark.parametrize('dtype', ['float16', 'bfloat16'])
 @pytest.mark.parametrize('dim', [64, 128])
 def test_prefill_ragged_key_splits(dtype, dim):
-    # A replacement batch of config-4 shape (16 heads): one long prompt among
-    # short ones. The long prompt's last tiles span more key blocks than their
-    # share of the launch, so their keys are split over workgroups and merged;
-    # every prompt against the oracle and the pool image bit for bit.
-    tokens, offsets = [1000, 60, 130, 5, 300], [0, 0, 20, 7, 0]
+    # One long prompt behind a long context among short ones, few heads: the
+    # launch leaves half the compute units idle, so the keys of the long
+    # prompt's tiles are split over workgroups and merged; every prompt against
+    # the oracle and the pool image bit for bit.
+    tokens, offsets = [1000, 60, 130, 5, 300], [1100, 0, 20, 7, 0]
     before = key_split_launches()
-    run_ragged(dtype, dim, tokens, offsets, h=16, seed=dim + 1)
+    run_ragged(dtype, dim, tokens, offsets, h=2, seed=dim + 1)
     assert key_split_launches() == before + 1, 'the ragged launch did not split the keys'
+    # the same prompts in a launch of 16 heads fill the compute units
+    run_ragged(dtype, dim, tokens, [0, 0, 20, 7, 0], h=16, seed=dim + 1)
+    assert key_split_launches() == before + 1
 
 
 def test_prefill_ragged_short_prompts_stay_unsplit():
