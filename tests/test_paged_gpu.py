@@ -353,23 +353,28 @@ def test_multi_token_append_and_causal_attention(dtype):
     assert_attention_close(out.to_numpy(), ref, dtype)
 
 
-@pytest.mark.parametrize('batch,columns', [(4, 64), (200, 64), (256, 64), (257, 64), (700, 64),
-                                           (2100, 64), (5, 160), (300, 160)])
-def test_decode_batch_device_ranked_order(batch, columns):
+@pytest.mark.parametrize('batch,heads,columns', [
+    (4, 3, 64), (256, 1, 64), (100, 3, 64), (200, 3, 64), (256, 3, 64),
+    (257, 17, 64), (700, 12, 64), (2048, 3, 64), (40, 35, 160), (300, 12, 160),
+    (257, 3, 64), (2100, 3, 64), (5, 3, 160), (300, 3, 160)])
+def test_decode_batch_device_ranked_order(batch, heads, columns):
     # Without a host work list mt_paged_decode_batch visits the rows longest
-    # first: b <= 256 rows of one split are ranked inside every workgroup;
-    # larger batches and tables that may split (160 columns: 2560 tokens, up
-    # to three splits) get a work list from order_kernel and a grid that
-    # strides over it; 2100 rows take batch order. Many equal lengths (ties
-    # go by row), an empty row (offset -1: zero output, no append) and a row
-    # past its table (NaN output, no append) keep every order a permutation:
-    # every (row, head) is written once, equal to the oracle, and the pool
-    # image matches bit for bit.
+    # first where there are more workgroups than compute units (256): b <= 256
+    # rows of one split are ranked inside every workgroup (100, 200 and 256 rows
+    # x 3 heads; 4 x 3 and 256 x 1 fit and take batch order). Larger batches and
+    # tables that may split (160 columns: 2560 tokens, three splits) get a work
+    # list from order_kernel and a grid that strides over it, from more than 16
+    # workgroups per compute unit on and up to 2048 rows: the second line of
+    # parameters, 4200 to 10800 workgroups beside the third line's, which take
+    # batch order. Many equal lengths (ties go by row), an empty row (offset -1:
+    # zero output, no append) and a row past its table (NaN output, no append)
+    # keep every order a permutation: every (row, head) is written once, equal
+    # to the oracle, and the pool image matches bit for bit.
     import dataclasses
     rng = np.random.default_rng([17, batch, columns])
     choices = [1, 16, 17, 64, 200, 1024] + ([1025, 2048, 2049, 2560] if columns > 64 else [])
     lengths = rng.choice(choices, size=batch)
-    case = make_decode_case(17, batch=batch, heads=3, dim=64, page_size=16, lengths=lengths,
+    case = make_decode_case(17, batch=batch, heads=heads, dim=64, page_size=16, lengths=lengths,
                             pool_pages=int(((lengths + 15) // 16).sum()) // 8 * 8 + 8, pages_per_slab=8,
                             dtype='float16', columns=columns)
     lengths = case.lengths.copy()

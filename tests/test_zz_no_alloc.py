@@ -76,6 +76,12 @@ def test_noalloc_matches_decode_batch_on_consecutive_calls():
     _compare(_case(4, batch=3, heads=2, dim=128, dtype='float32', max_len=2100))
 
 
+def test_noalloc_orders_a_large_batch_in_its_array():
+    # 130 rows x 12 heads x 3 splits, more than 16 workgroups per compute unit:
+    # the device-built visiting order lies in the array behind the partials
+    _compare(_case(5, batch=130, heads=12, dim=64, dtype='float16', max_len=3000))
+
+
 def test_noalloc_rejects_partials_beyond_its_array():
     # b*h = 32768 rows, 2 splits of d' = 128 partials: 34 MB > 32 MiB, refused
     # on the host before any launch. The arguments are real device buffers of
