@@ -1206,14 +1206,15 @@ struct QueryArgs {
   // Element strides of q and out per request, head and query: [b, h, nq, d]
   // by default, [b, nq, row] for head-interleaved token rows.
   int64_t q_b, q_h, q_r, o_b, o_h, o_r;
-  // The prompt's own K/V rows (strides of q), or null. When set (prefill
+  // The prompt's own K/V rows (strides of q), or null. When set (causal
   // kernel only), keys at or past the offset are read from these rows and the
   // workgroup of each query tile writes its tokens' K/V to their pages, which
   // replaces a separate append.
   const void* k;
   const void* v;
   // Key-split prefill: per (slot, head, query of the tile) D accumulators,
-  // max and denominator of one split's keys, merged by prefill_merge_kernel.
+  // max and denominator of one piece's keys, merged by uniform_merge_kernel or
+  // ragged_merge_kernel.
   float* partials;
 };
 
@@ -1534,8 +1535,8 @@ __device__ __forceinline__ float divided(float acc, float l, float inv) {
 }
 
 // What a staged row reads where there is nothing to read: NaN keys (a missing
-// page: its scores are NaN) and zeros.
-__device__ const uint32_t g_fill[8] = {~0u, ~0u, ~0u, ~0u, 0u, 0u, 0u, 0u};
+// page: its scores are NaN) and zeros, each a 16-byte load.
+__device__ __align__(16) const uint32_t g_fill[8] = {~0u, ~0u, ~0u, ~0u, 0u, 0u, 0u, 0u};
 
 // Copies 16 bytes per lane from global memory to LDS without passing through
 // registers: lane l's bytes land at lds + 16 l. The compiler does not see the
@@ -2987,7 +2988,7 @@ int mt_paged_prefill(void* out, const void* q, const void* k, const void* v, con
     if (e != hipErrorNotSupported) return e;
   }
   if (causal_kernel_takes(a, dtype) && aligned16(k) && aligned16(v)) {
-    // The prefill kernel reads the new keys from k/v and writes them to
+    // The causal kernel reads the new keys from k/v and writes them to
     // their pages itself: no separate append.
     a.k = k; a.v = v;
     return launch_query(a, dtype);
