@@ -4,6 +4,8 @@ separate pass), residual add fused with LayerNorm, and the strided head split
 that reads one column block of a fused QKV projection. References are numpy
 float64 restatements of the same math (tanh GELU of minitorch/nn.py:222-226,
 one-pass LayerNorm of src/layernorm_kernel.cu:37-99)."""
+import ctypes as ct
+
 import numpy as np
 import pytest
 
@@ -121,3 +123,20 @@ def test_heads_split_of_fused_qkv_block(dtype):
              b, n, h, d, 1, 3 * h * d, dtype_code(dtype))
         assert np.array_equal(out.to_numpy(), host[:, :, column].transpose(0, 2, 1, 3))
 
+
+
+def test_cast_to_bfloat16_bit_for_bit():
+    # Every upper half of a float32 (NaNs, infinities, subnormals and both zeros
+    # among them) with lower halves about the rounding's midpoint, against
+    # round-to-nearest-even with NaNs kept quiet.
+    from minitorch_amd.runtime import RawDeviceBuffer
+    from oracle import paged_oracle as po
+    low = np.array([0, 1, 0x7fff, 0x8000, 0x8001, 0xffff], np.uint32)
+    x = ((np.arange(65536, dtype=np.uint32)[:, None] << 16) | low).reshape(-1).view(np.float32)
+    src, dst = RawDeviceBuffer(x.nbytes), RawDeviceBuffer(2 * x.size)
+    src.upload(x)
+    call(model_library(), 'mt_cast', [P, P, ct.c_longlong, I, I], dst.ptr, src.ptr, x.size, dtype_code('float32'),
+         dtype_code('bfloat16'))
+    got, want = dst.download(np.uint16, x.size), po.bf16_encode(x)
+    bad = np.flatnonzero(got != want)
+    assert not len(bad), [(hex(x.view(np.uint32)[i]), hex(got[i]), hex(want[i])) for i in bad[:8]]
