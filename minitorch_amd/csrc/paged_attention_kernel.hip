@@ -1316,10 +1316,10 @@ struct AppendArgs {
 // P) between 12 MFMAs; rounds deeper in flight, and all loads through
 // registers, measured the same or slower. Against the 16-query waves with V
 // transposed by 2-byte LDS stores that it replaces (us per call, bf16): 2048
-// tokens at offset 2048 x 16 heads 60 against 134 (430 against 192 TFLOP/s),
-// 1000 tokens x 16 heads 15.2 against 22.7, 16 prompts of 32-512 tokens x 12
-// heads fp16 19.8 against 26.3; fp32, which query_kernel read K/V for once per
-// query: 4 x 333 tokens x 12 heads 20 against 106.
+// tokens at offset 2048 x 16 heads 59-65 by box against 134 (400-435 against 192
+// TFLOP/s), 1000 tokens x 16 heads 15.0 against 22.7, 16 prompts of 32-512 tokens
+// x 12 heads fp16 19.0-19.8 against 26.3; fp32, which query_kernel read K/V for
+// once per query: 4 x 333 tokens x 12 heads 22 against 106.
 //
 // For fp16/bf16 the MFMA takes P in the input type, so P is split into a high
 // and a low part of that type (two MFMAs): the weights keep about 16 (bf16)
@@ -1332,8 +1332,8 @@ struct AppendArgs {
 // are then at most 2^kRescale, which neither fp32 nor the hi/lo split minds.
 // fp16 has nothing below 2^-24, so its weights are taken 2^kHalfShift larger,
 // denominator and all: the split then keeps a weight's 22 bits down to 2^-11 of
-// the largest and ends at 2^-33 of it. At 2^-24, 1500 keys of weight 2^-18
-// beside one of weight 1 lost 1.4 % of their sum.
+// the largest and ends at 2^-33 of it. Ending at 2^-24, weights of 2.9e-6 beside
+// one of 1 in every block lost 1 % of their sum.
 constexpr int kPfWindowPages = 512;  // page bases resolved into LDS at a time
 constexpr int kPfBlock = 64;         // keys per unit of a split over workgroups
 constexpr float kRescale = 6.f;
@@ -2776,10 +2776,14 @@ struct CausalPlan {
 
 // tiles32/64/128: workgroups (tiles x heads, over all prompts) for tiles of
 // that many queries; blocks: key blocks of the longest tile; row_bytes: a K
-// row in LDS; queries: of the longest prompt. Where the lines lie (MI355X, 256 compute units, us per call):
+// row in LDS; queries: of the longest prompt; fp32: the type. Where the lines lie (MI355X, 256 compute units, us per call):
 // * kTiny and kShort for prompts of one and two key blocks, which end before
 //   wider workgroups have met: 8 x 100 tokens x 25 heads fp16 9.3 kShort
-//   against 11.5 kDense.
+//   against 11.5 kDense. Two blocks of a 16-bit type run kDeep while 64-query
+//   tiles take one round, whose eight waves stage and compute them at once: 16
+//   prompts of 20-60 tokens at offset 60 x 12 heads bf16 9.6 kShort and 8.7, 27
+//   of 31-62 at 29 18.7 and 16.6 (17.6 on the kernel before); in fp32 the two
+//   are within 3 % of each other either way.
 // * kNarrow while its workgroups take one round of the compute units (an
 //   eighth more still end with the long tiles): 300 tokens x 12 heads bf16 8.0
 //   against 8.8 kDeep, 700 x 12 fp32 (264 workgroups) 25.8 against 33.1; but
@@ -2799,12 +2803,12 @@ struct CausalPlan {
 //   narrow tiles leave half the compute units idle and the longest walks at
 //   least 8 rounds, in pieces of at least 3 (40 tokens at offset 4000 x 12
 //   heads bf16: 15.5 against 26.9).
-CausalPlan causal_plan(int64_t tiles32, int64_t tiles64, int64_t tiles128, int blocks, int row_bytes, int queries) {
+CausalPlan causal_plan(int64_t tiles32, int64_t tiles64, int64_t tiles128, int blocks, int row_bytes, int queries, bool fp32) {
   const int64_t cus = std::max(1, device_compute_units());
   CausalPlan plan{};
   const bool narrow = 8 * tiles32 <= 9 * cus || (queries <= 32 && row_bytes > 128);
   plan.config = blocks == 1             ? kTiny
-                : blocks == 2           ? kShort
+                : blocks == 2           ? (tiles64 <= cus && !fp32 ? kDeep : kShort)
                 : narrow                ? kNarrow
                 : tiles64 <= cus        ? kDeep
                 : 2 * tiles128 < 3 * cus ? kDense
@@ -2877,7 +2881,7 @@ hipError_t launch_query(QueryArgs& a, int dtype) {
     auto tiles = [&](int tq) { return (a.nq + tq - 1) / tq; };
     const int most = key_blocks(tiles(64) - 1, 64, a.nq, a.offset);
     const CausalPlan plan = causal_plan(bh * tiles(32), bh * tiles(64), bh * tiles(128), most,
-                                         (d <= 64 ? 64 : 128) * esize, a.nq);
+                                         (d <= 64 ? 64 : 128) * esize, a.nq, dtype == kF32);
     const int tq = config_queries(plan.config);
     UniformItems items{tiles(tq), 1, 0};
     if (plan.share > 0) {
@@ -3084,7 +3088,7 @@ int mt_paged_prefill_ragged(void* out, const void* q, const void* k, const void*
     // (narrow tiles only where the launch can list them)
     const CausalPlan plan = causal_plan(tiles32 <= kRaggedTiles ? tiles32 * h : INT64_MAX / 16, tiles64 * h,
                                         tiles128 * h, most, (d <= 64 ? 64 : 128) * int(e),
-                                        tiles32 <= kRaggedTiles ? queries : INT_MAX);
+                                        tiles32 <= kRaggedTiles ? queries : INT_MAX, dtype == kF32);
     const int tq = config_queries(plan.config);
     // (prompt, tile) pairs and their key blocks, the longest first; with a
     // share, cut into pieces of at most that many blocks as far as the
