@@ -34,7 +34,8 @@
 // Causal attention of several queries per request (a prefill) runs on the
 // matrix cores for every type and head dims of whole 16-byte chunks
 // (causal_kernel: 32 queries a wave, S^T = K Q^T and O^T += V^T P^T), a single
-// query on the decode kernel; other rows use the per-query query_kernel.
+// query on the decode kernel; other rows, and few queries where that is faster,
+// use the per-query query_kernel.
 #include "mt_device.h"
 #include "../../include/mt_paged.h"
 #include <algorithm>

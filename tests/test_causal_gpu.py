@@ -1,7 +1,10 @@
 """GPU parity of the matrix-core causal attention at the edges of its tiles and
 of its dispatch, against the float64 oracle: head dims that do not fill the
 kernel's 64 or 128 columns, fp32, query counts around the 32-, 64- and
-128-query tiles, every workgroup shape and keys split over workgroups.
+128-query tiles, every workgroup shape and keys split over workgroups; fp32's
+precision, small weights, and both sides of the lines to the per-query kernel
+(which the small fp32 grids of the tile edges run on at head dims 64 and 128;
+test_few_queries has the large ones).
 Tolerances are in tests/tolerances.py."""
 import numpy as np
 import pytest

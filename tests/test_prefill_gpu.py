@@ -2,8 +2,8 @@
 against the float64 oracle.
 
 Rows of whole, aligned 16-byte chunks run the matrix-core causal kernel (two
-or more queries) or the decode kernel (one); the others run the per-query
-kernel. All follow reference paged_forward with offsets == nullptr
+or more queries) or the decode kernel (one); the others, and few queries where
+it is faster (most small fp32 cases here), run the per-query kernel. All follow reference paged_forward with offsets == nullptr
 (src/paged_attention_kernel.cu:35-85): nk = offset + nq, query qi attends
 keys kj <= offset + qi, and a missing page gives NaN for every query that
 attends it. Page sizes are 8, 16 and 32 (the entry point rejects others). Tolerances are in tests/tolerances.py.
